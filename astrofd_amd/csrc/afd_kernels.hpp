@@ -1061,9 +1061,9 @@ AFD_D bool cell_c2p(const UpdArgs<F> &a, const double *U, bool live, long c, dou
             wave_enqueue(live && !done, c, a.queue, a.qcount, a.qcap);
             return done;
         }
-        if (live && !done) rmhd_c2p<FAST>(cp, U, q, st);
+        if (live && !done) rmhd_c2p<FAST>(cp, U, q, st, a.stats != nullptr);
     } else {
-        if (live) hydro_c2p<FAST>(a.gamma, a.gfac, a.p_max, a.v_max, U, q, st);
+        if (live) hydro_c2p<FAST>(a.gamma, a.gfac, a.p_max, a.v_max, U, q, st, a.stats != nullptr);
     }
     return live;
 }
@@ -1408,7 +1408,7 @@ template <typename F> __global__ __launch_bounds__(BLOCK) void k_c2p_queue(UpdAr
 #pragma unroll
         for (int v = 0; v < 9; ++v) U[v] = a.Uc[v * n + c];
         C2PStats sc = {0, 0, 0};
-        rmhd_c2p<sizeof(F) == 4>(cp, U, q, sc);
+        rmhd_c2p<sizeof(F) == 4>(cp, U, q, sc, a.stats != nullptr);
 #pragma unroll
         for (int v = 0; v < 9; ++v) a.Pout[v * n + c] = q[v];
         if (a.flags && a.stage == a.nst - 1) a.flags[c] = (unsigned char)sc.flags;

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_dataset(MlpDataArgs a) {
     rmhd_p2c_cell(a.gfac, a.p_max, a.v_max, q, U);
     RmhdC2PParams cp = {a.gamma, a.gfac, a.p_max, a.v_max};
     C2PStats st = {0, 0, 0};
-    rmhd_c2p(cp, U, out, st);
+    rmhd_c2p(cp, U, out, st, false);
     float x[5];
     bool ok = mlp_features(U, x);
     double v2 = out[1] * out[1] + out[2] * out[2] + out[3] * out[3];
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(BLOCK) void k_c2p_batch_learned(BatchArgs a, const 
     bool fok = mlp_features(U, x) && live;
     mlp_infer_wave(MlpGlobal{mlp_view(mlp)}, x, y);
     bool done = fok && rmhd_c2p_from_guess(cp, U, mlp_guess_Z(U[0], a.gfac, y), q, st);
-    if (live && !done) rmhd_c2p(cp, U, q, st);
+    if (live && !done) rmhd_c2p(cp, U, q, st, a.iters || a.stats);
     if (live) {
         for (int v = 0; v < 9; ++v) a.out[9 * m + v] = q[v];
         if (a.iters) a.iters[m] = st.hydro_iters + st.newton_iters;

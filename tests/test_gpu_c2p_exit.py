@@ -1,0 +1,72 @@
+"""The con2prim's early exit (hydro_c2p without iteration counts) against the full loop."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from astrofd_amd import _lib as L
+
+from .golden_states import smooth_state, srhd_state
+from .gpu_helpers import make_domain
+
+pytestmark = pytest.mark.gpu
+
+
+def conserved(physics, n, seed):
+    """Conserved states over wide ranges: cold to hot, static to W ~ 100, tau moved off its consistent
+    value by rounding, by the stopping tolerance and at random (both signs), D or S2 out of range."""
+    r = np.random.default_rng(seed)
+    kind = r.integers(0, 5, n)
+    rho = 10.0 ** r.uniform(-13, 6, n)
+    p = rho * 10.0 ** r.uniform(-14, 4, n)
+    W = 1.0 + 10.0 ** r.uniform(-17, 2, n)
+    D, w = rho * W, (rho + 2.5 * p) * W * W
+    S = w * np.sqrt(1.0 - 1.0 / W ** 2)
+    tau = w - p - D
+    tau = np.where(kind == 1, tau * (1.0 + 1e-15 * r.integers(-8, 9, n)), tau)
+    tau = np.where(kind == 2, tau + 10.0 ** r.uniform(-13, -9, n) * r.choice([-1.0, 1.0], n), tau)
+    tau = np.where(kind == 3, 10.0 ** r.uniform(-14, 5, n) * r.choice([-1.0, 1.0, 1.0], n), tau)
+    S = np.where(kind == 4, 10.0 ** r.uniform(-15, 5, n), S)
+    D = np.where(r.random(n) < 0.01, r.choice([0.0, -1e-3, 1e-14, np.nan, np.inf], n), D)
+    e = r.standard_normal((n, 3))
+    e /= np.linalg.norm(e, axis=1, keepdims=True)
+    U = np.zeros((n, 9 if physics == "rmhd" else 5))
+    U[:, 0], U[:, 1:4], U[:, 4] = D, S[:, None] * e, tau
+    if physics == "rmhd":
+        B = r.standard_normal((n, 3)) * (np.sqrt(np.abs(rho)) * 10.0 ** r.uniform(-3, 1, n))[:, None]
+        U[:, 5:8] = B
+        U[:, 4] += 0.5 * (B * B).sum(1)
+    return U
+
+
+@pytest.mark.parametrize("physics", ["hydro", "rmhd"])
+@pytest.mark.parametrize("p_max,v_max", [(1.0, 0.999), (1e4, 0.9999)])
+def test_batch_without_counts_is_the_counted_batch(physics, p_max, v_max):
+    nb = 9 if physics == "rmhd" else 5
+    U = conserved(physics, 100003, 5)
+    with make_domain(physics, (nb, 12, 12, 12), 2, p_max=p_max, v_max=v_max, gamma=4.0 / 3.0) as d:
+        ref, it = d.c2p(U, with_iters=True)
+        out = np.empty_like(ref)
+        L.check(d.lib.afd_c2p_batch(d.h, U.shape[0], L.dptr(U), L.dptr(out),
+                                    ctypes.POINTER(ctypes.c_int32)()), "afd_c2p_batch")
+    assert it.max() >= 30
+    assert np.array_equal(out, ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("physics", ["hydro", "rmhd"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_step_without_counters_is_the_counted_step(physics, precision):
+    shape = (21, 17, 23)
+    pr = smooth_state(shape, 3, physics, vamp=0.5)
+    if physics == "hydro":
+        pr[:, :, :, :11] = srhd_state(shape, 4)[:, :, :, :11]
+    outs = []
+    for stats in (False, True):
+        with make_domain(physics, pr.shape, 3, recon="weno", rk_order=3, precision=precision) as d:
+            d.set_prim(pr)
+            d.set_instrumentation(stats=stats)
+            for _ in range(2):
+                d.apply_bcs()
+                d.step(0.02)
+            outs.append(d.get_prim())
+    assert np.array_equal(outs[0], outs[1], equal_nan=True)

@@ -27,19 +27,21 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 # Packed FP32 VALU ops are disabled (-packed-fp32-ops): gfx950 code is written for scalar FP32/FP64.
 # MFMAs take their accumulators in ordinary VGPRs (-amdgpu-mfma-vgpr-form): with the accumulation
 # registers the network's forward kernel copied every result out with v_accvgpr_read (146 a wave)
-# and ran at 3 waves per SIMD instead of 5.
+# and ran at 3 waves per SIMD instead of 5.  (Not the training kernel: see afd_mlp_train.hip.)
 HIPFLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-Wall", "-Wno-unused-function",
             "-Wno-unused-variable", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-            "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-I", INCLUDE, "-I", CSRC]
+            "-I", INCLUDE, "-I", CSRC]
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 UNITS = [
-    ("afd_capi.hip", []),
-    ("afd_common.hip", []),
-    ("afd_srhd.hip", []),
-    ("afd_mlp.hip", []),
-    ("afd_fused.hip", []),
-    ("afd_rmhd.hip", ["-DAFD_RMHD_T=double"], "afd_rmhd_f64"),
-    ("afd_rmhd.hip", ["-DAFD_RMHD_T=float"], "afd_rmhd_f32"),
+    ("afd_capi.hip", VGPR_FORM),
+    ("afd_common.hip", VGPR_FORM),
+    ("afd_srhd.hip", VGPR_FORM),
+    ("afd_mlp.hip", VGPR_FORM),
+    ("afd_mlp_train.hip", []),
+    ("afd_fused.hip", VGPR_FORM),
+    ("afd_rmhd.hip", VGPR_FORM + ["-DAFD_RMHD_T=double"], "afd_rmhd_f64"),
+    ("afd_rmhd.hip", VGPR_FORM + ["-DAFD_RMHD_T=float"], "afd_rmhd_f32"),
 ]
 
 

@@ -1260,12 +1260,11 @@ extern "C" int afd_mlp_train(afd_ctx *c, int64_t steps, int32_t batch, float lr,
     if (batch <= 0 || batch > m.n_data) return fail(AFD_ERR_INVALID, "batch must be in [1, dataset size]");
     if (steps < 0 || steps > 65536) return fail(AFD_ERR_INVALID, "steps must be in [0, 65536] per call");
     HIPCHK(hipSetDevice(c->p.device));
+    if (!m.partial) ALLOC(c, m.partial, mlp_partial_bytes());
     const int64_t nbat = m.n_data / batch;
     for (int64_t st = 0; st < steps; ++st) {
         int64_t off = (st % nbat) * batch;
-        HIPCHK(mlp_loss_grad(m.w, m.X + 5 * off, m.Y + 2 * off, batch, m.grad, m.loss + st, c->stream));
-        HIPCHK(mlp_adam(m.master, m.adam_m, m.adam_v, m.grad, ++m.adam_t, lr, c->stream));
-        HIPCHK(mlp_pack(m.master, m.w, c->stream));
+        HIPCHK(mlp_train_step(m, m.X + 5 * off, m.Y + 2 * off, batch, lr, m.loss + st, c->stream));
     }
     if (loss_history && steps > 0)
         HIPCHK(hipMemcpyAsync(loss_history, m.loss, (size_t)steps * 8, hipMemcpyDeviceToHost, c->stream));
@@ -1303,6 +1302,7 @@ extern "C" int afd_mlp_loss_grad(afd_ctx *c, int64_t n, const float *X, const fl
     if (!c->mlp.loaded) return fail(AFD_ERR_STATE, "no weights loaded");
     if (n <= 0 || !X || !Y || !grad || !loss) return fail(AFD_ERR_INVALID, "afd_mlp_loss_grad: bad argument");
     HIPCHK(hipSetDevice(c->p.device));
+    if (!c->mlp.partial) ALLOC(c, c->mlp.partial, mlp_partial_bytes());
     float *dX = nullptr, *dY = nullptr;
     int rc = tmp_alloc(&dX, (size_t)n * 20);
     if (!rc) rc = tmp_alloc(&dY, (size_t)n * 8);
@@ -1310,7 +1310,7 @@ extern "C" int afd_mlp_loss_grad(afd_ctx *c, int64_t n, const float *X, const fl
     if (!rc) {
         e = hipMemcpyAsync(dX, X, (size_t)n * 20, hipMemcpyHostToDevice, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(dY, Y, (size_t)n * 8, hipMemcpyHostToDevice, c->stream);
-        if (e == hipSuccess) e = mlp_loss_grad(c->mlp.w, dX, dY, n, c->mlp.grad, c->mlp.loss, c->stream);
+        if (e == hipSuccess) e = mlp_loss_grad(c->mlp, dX, dY, n, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(grad, c->mlp.grad, MLP_NPARAM * 4, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(loss, c->mlp.loss, 8, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);

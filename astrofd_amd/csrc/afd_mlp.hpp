@@ -22,11 +22,18 @@ constexpr int MLP_OFF_W1 = 0, MLP_OFF_B1 = MLP_OFF_W1 + MLP_H * MLP_IN, MLP_OFF_
               MLP_OFF_B3 = MLP_OFF_W3 + MLP_OUT * MLP_H;
 constexpr size_t MLP_DEV_BYTES = (size_t)MLP_NBLK * 64 * 16 + (size_t)MLP_BIAS_FLOATS * 4;
 
+// A bias b as hi + lo: hi = the nearest BF16 of b, lo = the nearest BF16 of b - hi (exact in FP32).
+AFD_D float bias_part(float b, int which) {
+    const float hi = (float)(__bf16)b;
+    return which == 0 ? hi : b - hi;
+}
+
 struct MlpDevice {
     float *master = nullptr;   // MLP_NPARAM FP32
     void *w = nullptr;         // packed inference weights
     float *adam_m = nullptr, *adam_v = nullptr, *grad = nullptr;
     double *loss = nullptr;    // per training step
+    float *partial = nullptr;  // workgroups' partial gradients (mlp_partial_bytes), allocated by the first use
     float *X = nullptr, *Y = nullptr;  // dataset (n x 5 features, n x 2 targets)
     long n_data = 0, cap_data = 0;
     long adam_t = 0;
@@ -51,10 +58,11 @@ struct MlpDataArgs {
 };
 hipError_t mlp_prepare_dataset(const MlpDataArgs &a, hipStream_t s);
 hipError_t mlp_forward(const void *w, const float *X, long n, float *Y, hipStream_t s);
-// gradient of loss = mean over samples of sum over outputs (y - t)^2 accumulated into grad (zeroed here)
-hipError_t mlp_loss_grad(const void *w, const float *X, const float *Y, long n, float *grad, double *loss,
-                         hipStream_t s);
-hipError_t mlp_adam(float *master, float *m, float *v, const float *grad, long t, float lr, hipStream_t s);
+size_t mlp_partial_bytes();
+// gradient of loss = mean over samples of sum over outputs (y - t)^2 into d.grad, the loss into d.loss[0]
+hipError_t mlp_loss_grad(const MlpDevice &d, const float *X, const float *Y, long n, hipStream_t s);
+// one Adam step on the n samples: gradient, moments, master weights and their packed operands
+hipError_t mlp_train_step(MlpDevice &d, const float *X, const float *Y, long n, float lr, double *loss, hipStream_t s);
 hipError_t mlp_pack(const float *master, void *w, hipStream_t s);
 
 }  // namespace afd

@@ -39,6 +39,7 @@ UNITS = [
     ("afd_srhd.hip", VGPR_FORM),
     ("afd_mlp.hip", VGPR_FORM),
     ("afd_mlp_train.hip", []),
+    ("afd_xfer.hip", []),
     ("afd_fused.hip", VGPR_FORM),
     ("afd_rmhd.hip", VGPR_FORM + ["-DAFD_RMHD_T=double"], "afd_rmhd_f64"),
     ("afd_rmhd.hip", VGPR_FORM + ["-DAFD_RMHD_T=float"], "afd_rmhd_f32"),

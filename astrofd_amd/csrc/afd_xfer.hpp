@@ -1,0 +1,19 @@
+// afd_xfer.hpp -- host <-> device copies of whole arrays through pinned staging and a few host threads.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace afd {
+
+// One reference per context: the staging memory and the threads are made by the first large copy,
+// shared by every context of the process (any device), and given back with the last reference.
+void xfer_retain();
+void xfer_release();
+
+// Copy `bytes` between pageable host memory and device memory in stream order on `s` (a stream of the
+// current device) and wait for it: on return the host memory may be read or reused.
+hipError_t xfer_d2h(void *host, const void *dev, size_t bytes, hipStream_t s);
+hipError_t xfer_h2d(void *dev, const void *host, size_t bytes, hipStream_t s);
+
+}  // namespace afd

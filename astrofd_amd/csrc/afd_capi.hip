@@ -759,8 +759,6 @@ static int run_faces(afd_ctx *c, const double *P, bool skip_y = false) {
         for (int d = 0; d < 3; ++d) a.aux[d] = c->aux[d];
         a.rhs = c->rhs_pass;
         a.g = c->g;
-        a.physics = c->p.physics;
-        a.recon = c->p.recon_id;
         a.lim = c->p.limiter_id;
         a.np = c->p.n_passive;
         a.po = c->p.passive_offset;
@@ -768,8 +766,7 @@ static int run_faces(afd_ctx *c, const double *P, bool skip_y = false) {
         a.d[1] = c->p.dy;
         a.d[2] = c->p.dz;
         Timed t(c, 4);
-        hipLaunchKernelGGL(k_passive_rhs, grid1d(c->g.ncell), dim3(BLOCK), 0, c->stream, a);
-        HIPCHK(hipGetLastError());
+        HIPCHK(launch_passive_rhs(a, c->nb == 9, c->p.recon_id, c->stream));
     }
     return AFD_OK;
 }
@@ -888,14 +885,12 @@ extern "C" int afd_compute_rhs(afd_ctx *c, double *host, int64_t n) {
 static int run_sources(afd_ctx *c, SourceArgs &a) {
     if (!a.which) return AFD_OK;
     c->speed_valid = false;
-    const int ng = c->p.ng;
     a.P = c->P[c->cur];
     a.g = c->g;
-    a.ng = ng;
+    a.in = make_interior(c->g, c->p.ng);
     HIPCHK(hipSetDevice(c->p.device));
-    dim3 grid((unsigned)((long)c->p.nx * c->p.ny), (unsigned)((c->p.nz + BLOCK - 1) / BLOCK));
     Timed t(c, 4);
-    hipLaunchKernelGGL(k_sources, grid, dim3(BLOCK), 0, c->stream, a);
+    hipLaunchKernelGGL(k_sources, grid1d(a.in.count), dim3(BLOCK), 0, c->stream, a);
     HIPCHK(hipGetLastError());
     return AFD_OK;
 }
@@ -974,9 +969,9 @@ static int run_diss(afd_ctx *c, double dt, const afd_diss *d) {
     HIPCHK(hipSetDevice(c->p.device));
     // the new fields are staged in variable planes 5..14 of a primitive buffer the step is not using
     double *S = c->P[(c->cur + 1) % 3] + 5 * c->g.ncell;
-    DissArgs a{c->P[c->cur], S, c->g, c->p.ng, d->advect ? 1 : 0, dt, c->p.dx, c->p.dy, c->p.dz,
+    DissArgs a{c->P[c->cur], S, c->g, make_interior(c->g, c->p.ng), d->advect ? 1 : 0, dt, c->p.dx, c->p.dy, c->p.dz,
                d->zeta, d->eta, d->kappa, d->tau_bulk, d->tau_shear, d->tau_heat, d->cap_frac * d->p_max};
-    dim3 grid((unsigned)((long)c->p.nx * c->p.ny), (unsigned)((c->p.nz + BLOCK - 1) / BLOCK));
+    const dim3 grid = grid1d(a.in.count);
     Timed t(c, 4);
     hipLaunchKernelGGL(k_diss, grid, dim3(BLOCK), 0, c->stream, a);
     hipLaunchKernelGGL(k_diss_store, grid, dim3(BLOCK), 0, c->stream, a, c->P[c->cur]);

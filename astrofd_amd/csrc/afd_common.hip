@@ -4,51 +4,68 @@
 namespace afd {
 
 // ------------------------------------------------------------------ non-template kernels
-__global__ __launch_bounds__(BLOCK) void k_passive_rhs(PassiveArgs a) {
+// Which right-face variants the reference subtracts per direction, in the order WENO5 (bit 0), PPM
+// (bit 1), MUSCL (bit 2), and which variant's left flux survives; no variant: the direction has no term.
+enum { PASS_RMHD_MUSCL, PASS_SRHD_MUSCL, PASS_SRHD_PPM };
+template <int MODE> constexpr int pass_right(int dir) {
+    return MODE == PASS_RMHD_MUSCL ? 7 : (MODE == PASS_SRHD_MUSCL ? (dir == 0 ? 7 : (dir == 1 ? 0 : 4))
+                                                                  : (dir == 0 ? 0 : (dir == 1 ? 7 : 3)));
+}
+template <int MODE> constexpr int pass_left(int dir) { return MODE == PASS_SRHD_PPM && dir == 2 ? 1 : 2; }
+
+template <int MODE, int DIR>
+AFD_D void passive_dir(const PassiveArgs &a, const double *__restrict__ b, long c, const int *ijk, double &r) {
 #pragma clang fp contract(off)
-    const Grid &g = a.g;
-    long c = (long)blockIdx.x * BLOCK + threadIdx.x;
-    if (c >= g.ncell) return;
-    int i, j, k;
-    cell_ijk(g, c, i, j, k);
-    bool in = i >= g.r0[0] && i < g.r1[0] && j >= g.r0[1] && j < g.r1[1] && k >= g.r0[2] && k < g.r1[2];
-    for (int t = 0; t < a.np; ++t) {
-        double r = 0.0;
-        if (in) {
-            for (int dir = 0; dir < 3; ++dir) {
-                // which variants the reference evaluates per direction, and which left flux survives
-                int nvar;           // right-face variants subtracted, in order WENO, PPM, MUSCL
-                int vars[3];
-                int left;           // variant of the surviving left flux
-                if (a.physics == 1) {            // RMHD MUSCL: all three, every direction
-                    nvar = 3; vars[0] = 0; vars[1] = 1; vars[2] = 2; left = 2;
-                } else if (a.recon == 0) {       // SRHD MUSCL: x all three, y none, z MUSCL
-                    if (dir == 1) continue;
-                    if (dir == 0) { nvar = 3; vars[0] = 0; vars[1] = 1; vars[2] = 2; left = 2; }
-                    else { nvar = 1; vars[0] = 2; left = 2; }
-                } else {                         // SRHD PPM: x none, y all three, z WENO and PPM
-                    if (dir == 0) continue;
-                    if (dir == 1) { nvar = 3; vars[0] = 0; vars[1] = 1; vars[2] = 2; left = 2; }
-                    else { nvar = 2; vars[0] = 0; vars[1] = 1; left = 1; }
-                }
-                const double *ax = a.aux[dir];
-                long cp = c + (dir == 0 ? g.sx : (dir == 1 ? g.sy : 1L));
-                int ip = i + (dir == 0), jp = j + (dir == 1), kp = k + (dir == 2);
-                double sLa = ax[c], sRa = ax[g.ncell + c], vLa = ax[2 * g.ncell + c], vRa = ax[3 * g.ncell + c];
-                double sLb = ax[cp], sRb = ax[g.ncell + cp], vLb = ax[2 * g.ncell + cp], vRb = ax[3 * g.ncell + cp];
-                if (a.physics == 1) {  // right faces keep the left face's speeds (core/rmhd_core.py:915)
-                    sLb = sLa;
-                    sRb = sRa;
-                }
-                double FLt = passive_flux(a, left, a.po + t, dir, i, j, k, vLa, vRa, sLa, sRa);
-                for (int m = 0; m < nvar; ++m) {
-                    double FRt = passive_flux(a, vars[m], a.po + t, dir, ip, jp, kp, vLb, vRb, sLb, sRb);
-                    r -= (FRt - FLt) / a.d[dir];
-                }
-            }
+    constexpr int right = pass_right<MODE>(DIR);
+    if constexpr (right != 0) {
+        const Grid &g = a.g;
+        constexpr bool wide = (right & 3) != 0;  // WENO5 and PPM reach one cell further than MUSCL
+        const long s = dstride<DIR>(g);
+        const int n = DIR == 0 ? g.nx : (DIR == 1 ? g.ny : g.nz);
+        double q[7];
+#pragma unroll
+        for (int o = -3; o <= 3; ++o)
+            q[o + 3] = wide || (o >= -2 && o <= 2) ? b[c + pwrap(ijk[DIR], o, n) * s] : 0.0;
+        const double *ax = a.aux[DIR];
+        const long cp = c + s;
+        const double sLa = ax[c], sRa = ax[g.ncell + c], vLa = ax[2 * g.ncell + c], vRa = ax[3 * g.ncell + c];
+        const double vLb = ax[2 * g.ncell + cp], vRb = ax[3 * g.ncell + cp];
+        double sLb = sLa, sRb = sRa;
+        if (MODE != PASS_RMHD_MUSCL) {  // RMHD: right faces keep the left face's speeds (core/rmhd_core.py:915)
+            sLb = ax[cp];
+            sRb = ax[g.ncell + cp];
         }
-        a.rhs[t * g.ncell + c] = r;
+        const double FL = passive_flux<pass_left<MODE>(DIR)>(a.lim, q, vLa, vRa, sLa, sRa);
+        if (right & 1) r -= (passive_flux<0>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL) / a.d[DIR];
+        if (right & 2) r -= (passive_flux<1>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL) / a.d[DIR];
+        if (right & 4) r -= (passive_flux<2>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL) / a.d[DIR];
     }
+}
+
+template <int MODE> __global__ __launch_bounds__(BLOCK) void k_passive_rhs(PassiveArgs a) {
+    const Grid &g = a.g;
+    const long c = (long)blockIdx.x * BLOCK + threadIdx.x;
+    if (c >= g.ncell) return;
+    const int t = blockIdx.y;
+    int ijk[3];
+    cell_ijk(g, c, ijk[0], ijk[1], ijk[2]);
+    double r = 0.0;
+    if (in_range(g, c)) {
+        const double *b = a.P + (a.po + t) * g.ncell;
+        passive_dir<MODE, 0>(a, b, c, ijk, r);
+        passive_dir<MODE, 1>(a, b, c, ijk, r);
+        passive_dir<MODE, 2>(a, b, c, ijk, r);
+    }
+    a.rhs[t * g.ncell + c] = r;
+}
+
+// physics and recon: a context with passive fluxes (RMHD MUSCL, SRHD MUSCL or PPM)
+hipError_t launch_passive_rhs(const PassiveArgs &a, bool rmhd, int recon, hipStream_t s) {
+    const dim3 grid(grid1d(a.g.ncell).x, (unsigned)a.np);
+    if (rmhd) hipLaunchKernelGGL(k_passive_rhs<PASS_RMHD_MUSCL>, grid, dim3(BLOCK), 0, s, a);
+    else if (recon == 0) hipLaunchKernelGGL(k_passive_rhs<PASS_SRHD_MUSCL>, grid, dim3(BLOCK), 0, s, a);
+    else hipLaunchKernelGGL(k_passive_rhs<PASS_SRHD_PPM>, grid, dim3(BLOCK), 0, s, a);
+    return hipGetLastError();
 }
 
 __global__ __launch_bounds__(BLOCK) void k_c2p_batch(BatchArgs a) {
@@ -185,10 +202,8 @@ __device__ static double clamp01(double x, double lo, double hi) { return x < lo
 __global__ __launch_bounds__(BLOCK) void k_sources(SourceArgs a) {
 #pragma clang fp contract(off)
     const Grid &g = a.g;
-    const int nyi = g.ny - 2 * a.ng, nzi = g.nz - 2 * a.ng;
-    const int kk = blockIdx.y * BLOCK + threadIdx.x;
-    if (kk >= nzi) return;
-    const int i = a.ng + (int)blockIdx.x / nyi, j = a.ng + (int)blockIdx.x % nyi, k = a.ng + kk;
+    int i, j, k;
+    if (!interior_cell(g, a.in, i, j, k)) return;
     const long c = cidx(g, i, j, k), n = g.ncell;
     double *P = a.P;
     const double rho = P[c];
@@ -250,10 +265,8 @@ __global__ __launch_bounds__(BLOCK) void k_sources(SourceArgs a) {
 __global__ __launch_bounds__(BLOCK) void k_diss(DissArgs a) {
 #pragma clang fp contract(off)
     const Grid &g = a.g;
-    const int nyi = g.ny - 2 * a.ng, nzi = g.nz - 2 * a.ng;
-    const int kk = blockIdx.y * BLOCK + threadIdx.x;
-    if (kk >= nzi) return;
-    const int i = a.ng + (int)blockIdx.x / nyi, j = a.ng + (int)blockIdx.x % nyi, k = a.ng + kk;
+    int i, j, k;
+    if (!interior_cell(g, a.in, i, j, k)) return;
     const long c = cidx(g, i, j, k), n = g.ncell, sx = g.sx, sy = g.sy;
     const double *P = a.P;
     double f[10];
@@ -313,10 +326,8 @@ __global__ __launch_bounds__(BLOCK) void k_diss(DissArgs a) {
 
 __global__ __launch_bounds__(BLOCK) void k_diss_store(DissArgs a, double *P) {
     const Grid &g = a.g;
-    const int nyi = g.ny - 2 * a.ng, nzi = g.nz - 2 * a.ng;
-    const int kk = blockIdx.y * BLOCK + threadIdx.x;
-    if (kk >= nzi) return;
-    const int i = a.ng + (int)blockIdx.x / nyi, j = a.ng + (int)blockIdx.x % nyi, k = a.ng + kk;
+    int i, j, k;
+    if (!interior_cell(g, a.in, i, j, k)) return;
     const long c = cidx(g, i, j, k), n = g.ncell;
 #pragma unroll
     for (int m = 0; m < 10; ++m) P[(5 + m) * n + c] = a.S[m * n + c];

@@ -714,51 +714,93 @@ void k_face_rmhd_weno_march(FaceArgs<float> a) {
 // Passive fluxes of the reference's MUSCL (SRHD, RMHD) and PPM (SRHD) right-hand sides:
 // the face states of the WENO, PPM and MUSCL variants are recomputed here and combined with
 // the speeds/velocities the face kernels stored, in the reference's order of subtraction.
+// One thread per cell and passive (blockIdx.y), the scheme at compile time (k_passive_rhs<MODE>): the
+// seven values along an axis serve both faces and every variant, and the passives of a cell run side
+// by side.  (One thread walking all passives, each face and variant gathering its own six values with
+// a wrap test on each axis: 137 us for six passives on 64 x 60 x 66, now 48; one RMHD passive on
+// 75 x 66 x 81, 74 -> 36 us.)
 struct PassiveArgs {
     const double *P;
     const double *aux[3];   // per direction (sL, sR, vL, vR) x ncell
     double *rhs;            // n_passive x ncell, zero outside the range
     Grid g;
-    int physics, recon, lim, np, po;
+    int lim, np, po;
     double d[3];
 };
 
-AFD_D double pwrap(const Grid &g, const double *P, int v, int i, int j, int k) {
-    // Python negative-index wrap of the reference's passive stencils (i-3 at i = 2);
-    // indices past the end wrap as well (the reference reads out of range there).
-    if (i < 0) i += g.nx;
-    if (j < 0) j += g.ny;
-    if (k < 0) k += g.nz;
-    if (i >= g.nx) i -= g.nx;
-    if (j >= g.ny) j -= g.ny;
-    if (k >= g.nz) k -= g.nz;
-    return P[v * g.ncell + cidx(g, i, j, k)];
+// Offset (in cells along one axis) of position i + o of an axis of n cells: Python's negative-index
+// wrap of the reference's passive stencils (i - 3 at i = 2); positions past the end wrap as well
+// (the reference reads out of range there).
+AFD_D int pwrap(int i, int o, int n) {
+    int ii = i + o;
+    if (ii < 0) ii += n;
+    if (ii >= n) ii -= n;
+    return ii - i;
 }
 
-// variant 0 WENO5, 1 PPM, 2 MUSCL (core/srhd_core.py:554-580) on the face (c-1 | c)
-AFD_D double passive_flux(const PassiveArgs &a, int variant, int v, int dir, int i, int j, int k, double vL,
-                          double vR, double sL, double sR) {
-    double q[6];
-    for (int o = -3; o <= 2; ++o)
-        q[o + 3] = pwrap(a.g, a.P, v, i + (dir == 0 ? o : 0), j + (dir == 1 ? o : 0), k + (dir == 2 ? o : 0));
+// The passive face states and flux with every fused multiply-add written out.  Left to the compiler,
+// the choice of the product that is fused follows how often each product is used, so it changes with
+// the inlining of these functions; and PPM's edges jump where (qR - q0)(q0 - qL) changes sign, so
+// a last-bit change of a passive moves it by 1e-5 a few steps later.
+
+// WENO5 (core/srhd_core.py:343-377) on both sides of the face between q[2] and q[3]; the edge value from
+// the stencils qm2 .. qp2 given its three candidate polynomials
+AFD_D double passive_weno_edge(double qm2, double qm1, double q0, double qp1, double qp2, double p0, double p1,
+                               double p2) {
+#pragma clang fp contract(off)
+    const double eps = 1e-12, c = 13.0 / 12.0;
+    const double IS0 = fma(c, sq((qm2 - 2.0 * qm1) + q0), 0.25 * sq(fma(3.0, q0, qm2 - 4.0 * qm1)));
+    const double IS1 = fma(0.25, sq(qm1 - qp1), c * sq((qm1 - 2.0 * q0) + qp1));
+    const double IS2 = fma(c, sq((q0 - 2.0 * qp1) + qp2), 0.25 * sq(fma(-4.0, qp1, 3.0 * q0) + qp2));
+    const double a0 = 0.1 / sq(eps + IS0), a1 = 0.6 / sq(eps + IS1), a2 = 0.3 / sq(eps + IS2);
+    const double s = a0 + a1 + a2;
+    return fma(a2 / s, p2, fma(a0 / s, p0, (a1 / s) * p1));
+}
+AFD_D void passive_weno(const double *q, double &tL, double &tR) {
+#pragma clang fp contract(off)
+    const double c13 = 1.0 / 3.0, c76 = 7.0 / 6.0, c116 = 11.0 / 6.0, c56 = 5.0 / 6.0, c16 = 1.0 / 6.0;
+    tL = passive_weno_edge(q[0], q[1], q[2], q[3], q[4], fma(c116, q[2], fma(c13, q[0], -(c76 * q[1]))),
+                           fma(c13, q[3], fma(-c16, q[1], c56 * q[2])), fma(-c16, q[4], fma(c13, q[2], c56 * q[3])));
+    tR = passive_weno_edge(q[5], q[4], q[3], q[2], q[1], fma(c116, q[3], fma(c13, q[5], -(c76 * q[4]))),
+                           fma(c13, q[2], fma(c56, q[3], -c16 * q[4])), fma(-c16, q[1], fma(c13, q[3], c56 * q[2])));
+}
+
+// ppm_reconstruct with its two edge sums fused
+AFD_D void passive_ppm(double qm2, double qm1, double q0, double qp1, double qp2, double &oL, double &oR) {
+#pragma clang fp contract(off)
+    double qL = fma(7.0 / 12.0, qm1 + q0, -((1.0 / 12.0) * (qm2 + qp1)));
+    double qR = fma(7.0 / 12.0, q0 + qp1, -((1.0 / 12.0) * (qm1 + qp2)));
+    const double qmax = pymax(pymax(qm1, q0), qp1), qmin = pymin(pymin(qm1, q0), qp1);
+    if (qL > qmax) qL = qmax;
+    if (qL < qmin) qL = qmin;
+    if (qR > qmax) qR = qmax;
+    if (qR < qmin) qR = qmin;
+    if ((qR - q0) * (q0 - qL) <= 0.0) qL = qR = q0;
+    oL = qL;
+    oR = qR;
+}
+
+// The HLLE flux of one passive on the face between q[2] and q[3], from the face states of one
+// variant: 0 WENO5, 1 PPM, 2 MUSCL (core/srhd_core.py:554-580)
+template <int VARIANT>
+AFD_D double passive_flux(int lim, const double *q, double vL, double vR, double sL, double sR) {
+#pragma clang fp contract(off)
     double tL, tR;
-    if (variant == 0) {
-        tL = weno5_left<double>(q[0], q[1], q[2], q[3], q[4]);
-        tR = weno5_right<double>(q[5], q[4], q[3], q[2], q[1]);
-    } else if (variant == 1) {
+    if (VARIANT == 0) {
+        passive_weno(q, tL, tR);
+    } else if (VARIANT == 1) {
         double a0, b0;
-        ppm_reconstruct<double>(q[0], q[1], q[2], q[3], q[4], a0, tL);
-        ppm_reconstruct<double>(q[1], q[2], q[3], q[4], q[5], tR, b0);
+        passive_ppm(q[0], q[1], q[2], q[3], q[4], a0, tL);
+        passive_ppm(q[1], q[2], q[3], q[4], q[5], tR, b0);
     } else {
-        double slL = limiter<double>(a.lim, q[2] - q[1], q[3] - q[2]);
-        double slR = limiter<double>(a.lim, q[3] - q[2], q[4] - q[3]);
-        tL = q[2] + 0.5 * slL;
-        tR = q[3] - 0.5 * slR;
+        tL = q[2] + 0.5 * limiter<double>(lim, q[2] - q[1], q[3] - q[2]);
+        tR = q[3] - 0.5 * limiter<double>(lim, q[3] - q[2], q[4] - q[3]);
     }
-    return hlle_scalar<double>(tL, tR, tL * vL, tR * vR, sL, sR);
+    const double fL = tL * vL, fR = tR * vR;  // hlle_scalar
+    if (sL >= 0.0) return fL;
+    if (sR <= 0.0) return fR;
+    return fma(sL * sR, tR - tL, fma(sR, fL, -(sL * fR))) / (sR - sL + SMALL);
 }
-
-__global__ void k_passive_rhs(PassiveArgs a);
 
 // ------------------------------------------------------------------ stage update + c2p
 // Cells [lo, hi) per axis whose CFL speed a step's last stage takes: the flux range inside the
@@ -1469,13 +1511,36 @@ __global__ void k_nozzle(NozzleArgs a);
 // The driver's post-step sources (solvers/srhd3d_mpi_muscl.py:324-326), pointwise over the
 // interior, applied in that order to each cell in one pass: cooling/heating
 // (core/source_terms.py:5-28), two-temperature relaxation (:30-55), H/He ion chemistry
-// (core/chemistry.py:43-139).  One thread per cell of a k row; blockIdx.x = interior (i, j),
-// blockIdx.y = chunk of k.
+// (core/chemistry.py:43-139).  One thread per interior cell.
 enum { SRC_COOL = 1, SRC_TWO_TEMP = 2, SRC_CHEM = 4 };
+
+// The interior cells in order, k fastest, as a linear index: the last workgroup is the only partial one
+// whatever the extents.  (With one workgroup per k row and 256-cell chunk of it, a grid of 66 in z ran
+// with three quarters of its lanes idle: k_diss on 64 x 60 x 66 took 66 us, now 33.)
+struct Interior {
+    UDiv dk, dj;
+    unsigned nk, nj, count;
+    int ng;
+};
+inline Interior make_interior(const Grid &g, int ng) {
+    const unsigned nk = (unsigned)(g.nz - 2 * ng), nj = (unsigned)(g.ny - 2 * ng);
+    return Interior{make_udiv(nk), make_udiv(nj), nk, nj, nk * nj * (unsigned)(g.nx - 2 * ng), ng};
+}
+AFD_D bool interior_cell(const Grid &g, const Interior &in, int &i, int &j, int &k) {
+    const unsigned t = blockIdx.x * BLOCK + threadIdx.x;
+    if (t >= in.count) return false;
+    const unsigned r = udiv(in.dk, t), q = udiv(in.dj, r);
+    k = in.ng + (int)(t - r * in.nk);
+    j = in.ng + (int)(r - q * in.nj);
+    i = in.ng + (int)q;
+    return true;
+}
+
 struct SourceArgs {
     double *P;
     Grid g;
-    int ng, which;             // SRC_* bits
+    Interior in;
+    int which;                 // SRC_* bits
     double dt;
     double cool, heat, p_cap;  // COOLING_LAMBDA, HEATING_RATE, P_MAX
     int t_off;                 // Te, Ti
@@ -1492,7 +1557,8 @@ struct DissArgs {
     const double *P;
     double *S;
     Grid g;
-    int ng, advect;
+    Interior in;
+    int advect;
     double dt, dx, dy, dz;
     double zeta, eta, kappa, tau_bulk, tau_shear, tau_heat, cap;
 };

@@ -63,6 +63,9 @@ struct UpdLaunch {
 };
 hipError_t launch_update(const UpdLaunch &l, bool rhs_only, hipStream_t s);
 
+// Passive right-hand sides into a.rhs (contexts with passive fluxes: RMHD MUSCL, SRHD MUSCL and PPM).
+hipError_t launch_passive_rhs(const PassiveArgs &a, bool rmhd, int recon, hipStream_t s);
+
 // Mixed RMHD WENO5 on the flux-divergence path: the y faces fused with the stage update
 // (k_face_march_update), the ghost shell's update and the learned start's fallback queue.
 hipError_t launch_stage_fused(const FaceLaunch &l, const UpdLaunch &u, hipStream_t s);

@@ -65,6 +65,33 @@ template <bool FAST> AFD_D double dinvsqrt(double x) {  // 1 / sqrt(x), x > 0
     }
 }
 
+// Quotients by one divisor b, each rounded as a / b is.  FP64: the compiler's division scales numerator
+// and divisor together, so it refines the reciprocal again for every quotient (11 instructions); here
+// the refined reciprocal is shared and a quotient takes four (product, exact residual, correction and
+// the special cases), the same operations on the same values, so the same bits.  The scaling it leaves
+// out acts only near the ends of the exponent range: divisors are to lie in [2^-960, 2^960] (or be inf
+// or NaN), and quotients below 2^-970 may differ in their last bit.  FP32: the hardware reciprocal.
+template <typename T> struct Div;
+template <> struct Div<double> {
+    double b, y;
+    AFD_D explicit Div(double d) : b(d) {
+#pragma clang fp contract(off)
+        y = __builtin_amdgcn_rcp(d);
+        y = fma(y, fma(-d, y, 1.0), y);
+        y = fma(y, fma(-d, y, 1.0), y);
+    }
+    AFD_D double operator()(double a) const {
+#pragma clang fp contract(off)
+        const double q = a * y;
+        return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), y, q), b, a);
+    }
+};
+template <> struct Div<float> {
+    float b;
+    AFD_D explicit Div(float d) : b(d) {}
+    AFD_D float operator()(float a) const { return fdiv(a, b); }
+};
+
 template <typename T> AFD_D T pymin(T a, T b) { return (b < a) ? b : a; }
 template <typename T> AFD_D T sq(T x) { return x * x; }
 
@@ -239,10 +266,10 @@ AFD_D void hlle_vec(const T *UL, const T *UR, const T *FL, const T *FR, T sL, T 
 #pragma unroll
         for (int m = 0; m < N; ++m) out[m] = FR[m];
     } else {
-        T inv = sR - sL + Lim<T>::small;
+        const Div<T> by(sR - sL + Lim<T>::small);
         T sLsR = sL * sR;
 #pragma unroll
-        for (int m = 0; m < N; ++m) out[m] = fdiv(sR * FL[m] - sL * FR[m] + sLsR * (UR[m] - UL[m]), inv);
+        for (int m = 0; m < N; ++m) out[m] = by(sR * FL[m] - sL * FR[m] + sLsR * (UR[m] - UL[m]));
     }
 }
 
@@ -282,13 +309,13 @@ AFD_D void hllc5(const T *UL, const T *UR, const T *FL, const T *FR, T sL, T sR,
     const T *U = left ? UL : UR;
     const T *F = left ? FL : FR;
     T s = left ? sL : sR, p = left ? pL : pR, v = left ? vL : vR;
-    T den = s - sM + Lim<T>::small;
-    T fac = fdiv(s - v, den);
+    const Div<T> by(s - sM + Lim<T>::small);
+    T fac = by(s - v);
     T Ust[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) Ust[m] = U[m] * fac;
-    Ust[NM] = U[NM] * fac + fdiv(pStar - p, den);
-    Ust[4] = U[4] * fac + fdiv(pStar * sM - p * v, den);
+    Ust[NM] = U[NM] * fac + by(pStar - p);
+    Ust[4] = U[4] * fac + by(pStar * sM - p * v);
 #pragma unroll
     for (int m = 0; m < 5; ++m) out[m] = F[m] + s * (Ust[m] - U[m]);
     if constexpr (sizeof(T) == 4) {
@@ -398,9 +425,17 @@ template <typename T, bool FAST = false> AFD_D void rmhd_p2c_W(const Phys<T> &ph
     T rhoh = rho * h;
     T vb = vx * Bx + vy * By + vz * Bz;
     T b0 = W * vb;
-    T bx = dv(Bx + b0 * vx, W);
-    T by = dv(By + b0 * vy, W);
-    T bz = dv(Bz + b0 * vz, W);
+    T bx, by, bz;
+    if constexpr (FAST) {
+        bx = dv(Bx + b0 * vx, W);
+        by = dv(By + b0 * vy, W);
+        bz = dv(Bz + b0 * vz, W);
+    } else {
+        const Div<T> byW(W);
+        bx = byW(Bx + b0 * vx);
+        by = byW(By + b0 * vy);
+        bz = byW(Bz + b0 * vz);
+    }
     T b2 = (bx * bx + by * by + bz * bz) - b0 * b0;
     T rhohWW = rhoh * W * W;
     T wtot = rhohWW + B2;
@@ -449,9 +484,10 @@ template <typename T> AFD_D T rmhd_fast_speed_W(const Phys<T> &ph, const T *q, T
     T rhoh = rho * h;
     T vb = vx * Bx + vy * By + vz * Bz;
     T b0 = W * vb;
-    T bx = fdiv(Bx + b0 * vx, W);
-    T by = fdiv(By + b0 * vy, W);
-    T bz = fdiv(Bz + b0 * vz, W);
+    const Div<T> byW(W);
+    T bx = byW(Bx + b0 * vx);
+    T by = byW(By + b0 * vy);
+    T bz = byW(Bz + b0 * vz);
     T b2 = (bx * bx + by * by + bz * bz) - b0 * b0;
     T cs2 = fdiv(ph.gamma * p, pymax(rhoh, Lim<T>::small));
     if (cs2 < T(0)) cs2 = T(0);
@@ -684,9 +720,10 @@ AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const do
         if (p > p_max) p = p_max;
     }
     double Wm = E + p;
-    double vx = Sx / pymax(Wm, SMALL);
-    double vy = Sy / pymax(Wm, SMALL);
-    double vz = Sz / pymax(Wm, SMALL);
+    const Div<double> byWm(pymax(Wm, SMALL));
+    double vx = byWm(Sx);
+    double vy = byWm(Sy);
+    double vz = byWm(Sz);
     double v2 = vx * vx + vy * vy + vz * vz;
     if (v2 >= vmax2) {
         double fac = v_max / sqrt(v2 + 1e-32);
@@ -762,10 +799,18 @@ AFD_D bool rmhd_recover(const RmhdC2PParams &c, double Z, const double *U, doubl
     double Sx = U[1], Sy = U[2], Sz = U[3], D = U[0], Bx = U[5], By = U[6], Bz = U[7];
     double ZpB = Z + B2;
     double vb = ddiv<FAST>(SB, pymax(Z, SMALL));
-    double rZ = ddiv<FAST>(1.0, pymax(ZpB, SMALL));
-    double vx = FAST ? (Sx + vb * Bx) * rZ : (Sx + vb * Bx) / pymax(ZpB, SMALL);
-    double vy = FAST ? (Sy + vb * By) * rZ : (Sy + vb * By) / pymax(ZpB, SMALL);
-    double vz = FAST ? (Sz + vb * Bz) * rZ : (Sz + vb * Bz) / pymax(ZpB, SMALL);
+    double vx, vy, vz;
+    if constexpr (FAST) {
+        double rZ = ddiv<FAST>(1.0, pymax(ZpB, SMALL));
+        vx = (Sx + vb * Bx) * rZ;
+        vy = (Sy + vb * By) * rZ;
+        vz = (Sz + vb * Bz) * rZ;
+    } else {
+        const Div<double> byZ(pymax(ZpB, SMALL));
+        vx = byZ(Sx + vb * Bx);
+        vy = byZ(Sy + vb * By);
+        vz = byZ(Sz + vb * Bz);
+    }
     double v2 = vx * vx + vy * vy + vz * vz;
     double vmax2 = c.v_max * c.v_max;
     if (v2 >= vmax2) {

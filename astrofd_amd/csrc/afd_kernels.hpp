@@ -1008,12 +1008,13 @@ template <int NB, typename F> AFD_D void cell_rhs_flat(const UpdArgs<F> &a, long
 #pragma clang fp contract(off)
     const Grid &g = a.g;
     if constexpr (sizeof(F) == 8) {  // FP64 path: the reference's divisions
+        const Div<double> bx(a.dx), by(a.dy), bz(a.dz);
 #pragma unroll
         for (int v = 0; v < NB; ++v) {
             long o = v * g.ncell + c;
-            rhs[v] -= ((double)a.Fx[o + g.sx] - (double)a.FxL[o]) / a.dx;
-            rhs[v] -= ((double)a.Fy[o + g.sy] - (double)a.Fy[o]) / a.dy;
-            rhs[v] -= ((double)a.Fz[o + 1] - (double)a.Fz[o]) / a.dz;
+            rhs[v] -= bx((double)a.Fx[o + g.sx] - (double)a.FxL[o]);
+            rhs[v] -= by((double)a.Fy[o + g.sy] - (double)a.Fy[o]);
+            rhs[v] -= bz((double)a.Fz[o + 1] - (double)a.Fz[o]);
         }
     } else if (a.D) {  // the face kernels accumulated the divergence, already over the spacings
 #pragma unroll

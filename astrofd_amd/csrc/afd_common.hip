@@ -35,10 +35,11 @@ AFD_D void passive_dir(const PassiveArgs &a, const double *__restrict__ b, long 
             sLb = ax[cp];
             sRb = ax[g.ncell + cp];
         }
+        const Div<double> by(a.d[DIR]);
         const double FL = passive_flux<pass_left<MODE>(DIR)>(a.lim, q, vLa, vRa, sLa, sRa);
-        if (right & 1) r -= (passive_flux<0>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL) / a.d[DIR];
-        if (right & 2) r -= (passive_flux<1>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL) / a.d[DIR];
-        if (right & 4) r -= (passive_flux<2>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL) / a.d[DIR];
+        if (right & 1) r -= by(passive_flux<0>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL);
+        if (right & 2) r -= by(passive_flux<1>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL);
+        if (right & 4) r -= by(passive_flux<2>(a.lim, q + 1, vLb, vRb, sLb, sRb) - FL);
     }
 }
 
@@ -274,15 +275,15 @@ __global__ __launch_bounds__(BLOCK) void k_diss(DissArgs a) {
     for (int m = 0; m < 10; ++m) f[m] = P[(5 + m) * n + c];
     const double vx = P[n + c], vy = P[2 * n + c], vz = P[3 * n + c];
     if (a.advect) {  // core/dissipation.py:60-92, first-order upwind with the cell's velocity
-        const double hx = pymax(a.dx, 1e-12), hy = pymax(a.dy, 1e-12), hz = pymax(a.dz, 1e-12);
+        const Div<double> hx(pymax(a.dx, 1e-12)), hy(pymax(a.dy, 1e-12)), hz(pymax(a.dz, 1e-12));
         const long ox = vx > 0.0 ? -sx : sx, oy = vy > 0.0 ? -sy : sy, oz = vz > 0.0 ? -1 : 1;
 #pragma unroll
         for (int m = 0; m < 10; ++m) {
             const double *q = P + (5 + m) * n + c;
             const double u0 = f[m];
-            double dudx = vx > 0.0 ? (u0 - q[ox]) / hx : (q[ox] - u0) / hx;
-            double dudy = vy > 0.0 ? (u0 - q[oy]) / hy : (q[oy] - u0) / hy;
-            double dudz = vz > 0.0 ? (u0 - q[oz]) / hz : (q[oz] - u0) / hz;
+            double dudx = hx(vx > 0.0 ? u0 - q[ox] : q[ox] - u0);
+            double dudy = hy(vy > 0.0 ? u0 - q[oy] : q[oy] - u0);
+            double dudz = hz(vz > 0.0 ? u0 - q[oz] : q[oz] - u0);
             f[m] = u0 - a.dt * (vx * dudx + vy * dudy + vz * dudz);
         }
     }
@@ -296,28 +297,31 @@ __global__ __launch_bounds__(BLOCK) void k_diss(DissArgs a) {
     auto clamp = [cap](double x) { return x > cap ? cap : (x < -cap ? -cap : x); };
     if (a.zeta != 0.0) {  // bulk, :122-130
         double pi_eq = -a.zeta * divv;
-        f[0] = clamp((f[0] + a.dt * pi_eq / a.tau_bulk) / (1.0 + a.dt / a.tau_bulk));
+        const Div<double> tau(a.tau_bulk), den(1.0 + tau(a.dt));
+        f[0] = clamp(den(f[0] + tau(a.dt * pi_eq)));
     }
     if (a.eta != 0.0) {  // shear, :132-177 (pi^zz reset to -(pi^xx + pi^yy) before the caps)
-        const double third = 1.0 / 3.0, m2e = -2.0 * a.eta, ts = a.tau_shear;
+        const double third = 1.0 / 3.0, m2e = -2.0 * a.eta;
+        const Div<double> tau(a.tau_shear), den(1.0 + tau(a.dt));
         const double e[6] = {m2e * (dvx_dx - third * divv), m2e * (dvy_dy - third * divv),
                              m2e * (dvz_dz - third * divv), m2e * (0.5 * (dvx_dy + dvy_dx)),
                              m2e * (0.5 * (dvx_dz + dvz_dx)), m2e * (0.5 * (dvy_dz + dvz_dy))};
         double s6[6];
 #pragma unroll
-        for (int m = 0; m < 6; ++m) s6[m] = (f[1 + m] + a.dt * e[m] / ts) / (1.0 + a.dt / ts);
+        for (int m = 0; m < 6; ++m) s6[m] = den(f[1 + m] + tau(a.dt * e[m]));
         s6[2] = -(s6[0] + s6[1]);
 #pragma unroll
         for (int m = 0; m < 6; ++m) f[1 + m] = clamp(s6[m]);
     }
     if (a.kappa != 0.0) {  // heat flux, :179-213, T = p / max(rho, 1e-12)
         const double *R = P + c, *Pp = P + 4 * n + c;
-        auto T = [&](long o) { return Pp[o] / pymax(R[o], 1e-12); };
+        const Div<double> tau(a.tau_heat), den(1.0 + tau(a.dt));
+        auto T = [&](long o) { return fdiv(Pp[o], pymax(R[o], 1e-12)); };
         const double g3[3] = {(T(sx) - T(-sx)) * i2x, (T(sy) - T(-sy)) * i2y, (T(1) - T(-1)) * i2z};
 #pragma unroll
         for (int m = 0; m < 3; ++m) {
             double q_eq = -a.kappa * g3[m];
-            f[7 + m] = clamp((f[7 + m] + a.dt * q_eq / a.tau_heat) / (1.0 + a.dt / a.tau_heat));
+            f[7 + m] = clamp(den(f[7 + m] + tau(a.dt * q_eq)));
         }
     }
 #pragma unroll

@@ -35,42 +35,17 @@ template <typename T> struct Phys {
 };
 
 template <typename T> AFD_D T pymax(T a, T b) { return (b > a) ? b : a; }
-// Division and square root in the compute type: IEEE in FP64 (the plain path rounds as the
-// reference); in the FP32 path the hardware reciprocal and square root (about 1 ulp), whose
-// error is far below the FP32 rounding the mixed path already accepts.
-template <typename T> AFD_D T fdiv(T a, T b) { return a / b; }
-template <> AFD_D float fdiv<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-template <typename T> AFD_D T fsqrt(T x) { return sqrt(x); }
-template <> AFD_D float fsqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
-// FP64 division / inverse square root.  FAST = false: IEEE (the plain path rounds as the
-// reference).  FAST = true (mixed path: con2prim, Lorentz factors): the hardware reciprocal / reciprocal square
-// root refined by one Newton step (measured on gfx950: <= 11 ulp for 1/x, <= 20 ulp for 1/sqrt x),
-// at about a third of the instructions.  Newton-update divisions and the rare cap branches stay IEEE in both.
-template <bool FAST> AFD_D double ddiv(double a, double b) {
-    if constexpr (FAST) {
-        double r = __builtin_amdgcn_rcp(b);
-        r = fma(r, fma(-b, r, 1.0), r);
-        return a * r;
-    } else {
-        return a / b;
-    }
-}
-template <bool FAST> AFD_D double dinvsqrt(double x) {  // 1 / sqrt(x), x > 0
-    if constexpr (FAST) {
-        double y = __builtin_amdgcn_rsq(x);
-        double h = 0.5 * x * y;
-        return y * fma(-h, y, 1.5);
-    } else {
-        return 1.0 / sqrt(x);
-    }
-}
-
 // Quotients by one divisor b, each rounded as a / b is.  FP64: the compiler's division scales numerator
-// and divisor together, so it refines the reciprocal again for every quotient (11 instructions); here
-// the refined reciprocal is shared and a quotient takes four (product, exact residual, correction and
-// the special cases), the same operations on the same values, so the same bits.  The scaling it leaves
-// out acts only near the ends of the exponent range: divisors are to lie in [2^-960, 2^960] (or be inf
-// or NaN), and quotients below 2^-970 may differ in their last bit.  FP32: the hardware reciprocal.
+// and divisor first and refines the reciprocal for every quotient (11 instructions); here the refined
+// reciprocal is shared, a quotient takes four (product, exact residual, correction and the special
+// cases) and nothing is scaled: the same operations on the same values, so the same bits.  The scaling
+// acts only near the ends of the exponent range: divisors are to lie in [2^-960, 2^1020] (or be 0, inf
+// or NaN), quotients below 2^-970 may differ in their last bit and one beyond the largest double is NaN,
+// not inf.  Every FP64 division and square root of the physics goes through Div, fsqrt and finvsqrt: the
+// FP64 kernels are bound by vector instructions, of which the scaling was a tenth (RMHD WENO5 faces of a
+// 160^3 grid: 385, 358 and 344 us with it, 333, 303 and 286 without; SRHD MUSCL faces at 256^3: 498 and
+// 472 us).  FP32: the hardware reciprocal (about 1 ulp), whose error is far below the FP32 rounding the
+// mixed path already accepts.
 template <typename T> struct Div;
 template <> struct Div<double> {
     double b, y;
@@ -89,8 +64,65 @@ template <> struct Div<double> {
 template <> struct Div<float> {
     float b;
     AFD_D explicit Div(float d) : b(d) {}
-    AFD_D float operator()(float a) const { return fdiv(a, b); }
+    AFD_D float operator()(float a) const { return a * __builtin_amdgcn_rcpf(b); }
 };
+// Division in the compute type, as Div: FP64 as IEEE, so the plain path rounds as the reference
+template <typename T> AFD_D T fdiv(T a, T b) { return Div<T>(b)(a); }
+
+// Square root.  FP64: sqrt(x) rounded as the compiler's, except for 0 < x < 2^-760, whose scaling it
+// leaves out: Goldschmidt's iteration on the hardware's 1 / sqrt(x) (Markstein, "IA-64 and Elementary
+// Functions", ch. 9), two corrections by the exact residual, and div_fixup for 0, inf and NaN; 11
+// instructions for 18.  h is half of 1 / sqrt(x) to 2^-45.  FP32: the hardware's (about 1 ulp).
+AFD_D double sqrt_core(double x, double &h) {
+#pragma clang fp contract(off)
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y;
+    h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+}
+template <typename T> AFD_D T fsqrt(T x) {
+    double h;
+    const double g = sqrt_core(x, h);
+    return __builtin_amdgcn_div_fixup(g, 1.0, x);
+}
+template <> AFD_D float fsqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
+// 1 / sqrt(x) rounded as 1.0 / sqrt(x) is (both operations), same x: the reciprocal's refinement starts
+// from the root's h, not from another hardware reciprocal.  It starts an ulp high: 1 / g of the largest g
+// below a power of two lies just above a midpoint, which a start from below never leaves.
+AFD_D double finvsqrt(double x) {
+#pragma clang fp contract(off)
+    double h;
+    const double g = sqrt_core(x, h);
+    double y = h * (2.0 + 0x1p-51);
+    y = fma(y, fma(-g, y, 1.0), y);
+    return __builtin_amdgcn_div_fixup(fma(fma(-g, y, 1.0), y, y), x, 1.0);
+}
+// FP64 division / inverse square root.  FAST = false: IEEE (the plain path rounds as the
+// reference).  FAST = true (mixed path: con2prim, Lorentz factors): the hardware reciprocal / reciprocal square
+// root refined by one Newton step (measured on gfx950: <= 11 ulp for 1/x, <= 20 ulp for 1/sqrt x),
+// at about a third of the instructions.  Newton-update divisions and the rare cap branches stay IEEE in both.
+template <bool FAST> AFD_D double ddiv(double a, double b) {
+    if constexpr (FAST) {
+        double r = __builtin_amdgcn_rcp(b);
+        r = fma(r, fma(-b, r, 1.0), r);
+        return a * r;
+    } else {
+        return fdiv(a, b);
+    }
+}
+template <bool FAST> AFD_D double dinvsqrt(double x) {  // 1 / sqrt(x), x > 0
+    if constexpr (FAST) {
+        double y = __builtin_amdgcn_rsq(x);
+        double h = 0.5 * x * y;
+        return y * fma(-h, y, 1.5);
+    } else {
+        return finvsqrt(x);
+    }
+}
 
 template <typename T> AFD_D T pymin(T a, T b) { return (b < a) ? b : a; }
 template <typename T> AFD_D T sq(T x) { return x * x; }
@@ -142,25 +174,38 @@ template <typename T> AFD_D void ppm_reconstruct(T qm2, T qm1, T q0, T qp1, T qp
     oR = qR;
 }
 
-// core/srhd_core.py:343-359 (WENO5-JS, Jiang & Shu 1996, eps = 1e-12, weights 0.1/0.6/0.3)
-template <typename T> AFD_D T weno5_left(T qm2, T qm1, T q0, T qp1, T qp2) {
+// core/srhd_core.py:343-359 (WENO5-JS, Jiang & Shu 1996, eps = 1e-12, weights 0.1/0.6/0.3).  The FP64
+// indicators have every fused multiply-add written out: left to the compiler, which product is fused
+// follows what the neighbouring edges share, so a change elsewhere in a kernel would move its results by
+// an ulp.  fuse3: the product of 3 q0 - 4 qp1 that is fused (both are exact to an ulp).
+template <typename T>
+AFD_D void weno5_indicators(T qm2, T qm1, T q0, T qp1, T qp2, bool fuse3, T &IS0, T &IS1, T &IS2) {
+#pragma clang fp contract(off)
+    static_assert(sizeof(T) == 8, "the FP32 edges have their own");
+    const T c = 13.0 / 12.0;
+    IS0 = fma(c, sq(fma(-2.0, qm1, qm2) + q0), 0.25 * sq(fma(3.0, q0, fma(-4.0, qm1, qm2))));
+    IS1 = fma(0.25, sq(qm1 - qp1), c * sq(fma(-2.0, q0, qm1) + qp1));
+    const T d = fuse3 ? fma(3.0, q0, -(4.0 * qp1)) : fma(-4.0, qp1, 3.0 * q0);
+    IS2 = fma(c, sq(fma(-2.0, qp1, q0) + qp2), 0.25 * sq(d + qp2));
+}
+template <typename T> AFD_D T weno5_left(T qm2, T qm1, T q0, T qp1, T qp2, bool fuse3) {
     const T eps = T(1e-12);
-    T IS0 = T(13.0 / 12.0) * sq(qm2 - T(2) * qm1 + q0) + T(0.25) * sq(qm2 - T(4) * qm1 + T(3) * q0);
-    T IS1 = T(13.0 / 12.0) * sq(qm1 - T(2) * q0 + qp1) + T(0.25) * sq(qm1 - qp1);
-    T IS2 = T(13.0 / 12.0) * sq(q0 - T(2) * qp1 + qp2) + T(0.25) * sq(T(3) * q0 - T(4) * qp1 + qp2);
+    T IS0, IS1, IS2;
+    weno5_indicators(qm2, qm1, q0, qp1, qp2, fuse3, IS0, IS1, IS2);
     T a0 = fdiv(T(0.1), sq(eps + IS0));
     T a1 = fdiv(T(0.6), sq(eps + IS1));
     T a2 = fdiv(T(0.3), sq(eps + IS2));
     T s = a0 + a1 + a2;
-    T w0 = fdiv(a0, s), w1 = fdiv(a1, s), w2 = fdiv(a2, s);
+    const Div<T> by(s);
+    T w0 = by(a0), w1 = by(a1), w2 = by(a2);
     T p0 = T(1.0 / 3.0) * qm2 - T(7.0 / 6.0) * qm1 + T(11.0 / 6.0) * q0;
     T p1 = T(-1.0 / 6.0) * qm1 + T(5.0 / 6.0) * q0 + T(1.0 / 3.0) * qp1;
     T p2 = T(1.0 / 3.0) * q0 + T(5.0 / 6.0) * qp1 - T(1.0 / 6.0) * qp2;
     return w0 * p0 + w1 * p1 + w2 * p2;
 }
 // core/srhd_core.py:361-377 (mirror image)
-template <typename T> AFD_D T weno5_right(T qp2, T qp1, T q0, T qm1, T qm2) {
-    return weno5_left(qp2, qp1, q0, qm1, qm2);
+template <typename T> AFD_D T weno5_right(T qp2, T qp1, T q0, T qm1, T qm2, bool fuse3) {
+    return weno5_left(qp2, qp1, q0, qm1, qm2, fuse3);
 }
 
 // FP32 WENO5 of large deviations.  The nonlinear weights a_k / sum(a_j) with a_k = c_k / (eps + IS_k)^2
@@ -346,7 +391,7 @@ AFD_D void srhd_floor(double p_max, double v_max, double *q) {
     if (q[4] > p_max) q[4] = p_max;
     double v2 = q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
     if (v2 >= v_max * v_max) {
-        double fac = v_max / sqrt(v2 + 1e-32);
+        double fac = fdiv(v_max, fsqrt(v2 + 1e-32));
         q[1] *= fac;
         q[2] *= fac;
         q[3] *= fac;
@@ -398,7 +443,7 @@ template <bool FAST = false> AFD_D double rmhd_cap_W(double v_max, const double 
     double vx = q[1], vy = q[2], vz = q[3];
     double v2 = vx * vx + vy * vy + vz * vz;
     if (v2 >= v_max * v_max) {
-        double fac = v_max / sqrt(v2 + 1e-32);
+        double fac = fdiv(v_max, fsqrt(v2 + 1e-32));
         vx *= fac;
         vy *= fac;
         vz *= fac;
@@ -726,15 +771,15 @@ AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const do
     double vz = byWm(Sz);
     double v2 = vx * vx + vy * vy + vz * vz;
     if (v2 >= vmax2) {
-        double fac = v_max / sqrt(v2 + 1e-32);
+        double fac = fdiv(v_max, fsqrt(v2 + 1e-32));
         vx *= fac;
         vy *= fac;
         vz *= fac;
     }
     v2 = vx * vx + vy * vy + vz * vz;
     if (v2 >= 1.0) v2 = 1.0 - 1e-14;
-    double W = 1.0 / sqrt(1.0 - v2);
-    double rho = D / pymax(W, SMALL);
+    double W = finvsqrt(1.0 - v2);
+    double rho = fdiv(D, pymax(W, SMALL));
     if (rho < SMALL) rho = SMALL;
     if (p < SMALL) p = SMALL;
     if (p > p_max) p = p_max;
@@ -759,10 +804,10 @@ AFD_D double rmhd_f_of_Z(const RmhdC2PParams &c, double Z, double D, double tau,
     double vmax2 = c.v_max * c.v_max;
     if (v2 >= vmax2) v2 = vmax2 - 1e-14;
     double W2 = ddiv<FAST>(1.0, 1.0 - v2);
-    double W = FAST ? 1.0 * dinvsqrt<FAST>(1.0 - v2) : sqrt(W2);
+    double W = FAST ? 1.0 * dinvsqrt<FAST>(1.0 - v2) : fsqrt(W2);
     double rho = ddiv<FAST>(D, pymax(W, SMALL));
     double h = ddiv<FAST>(Z, pymax(rho * W2, SMALL));
-    double p = (h - 1.0) * rho * (c.gamma - 1.0) / c.gamma;
+    double p = fdiv((h - 1.0) * rho * (c.gamma - 1.0), c.gamma);
     if (p < SMALL) p = SMALL;
     if (p > c.p_max) p = c.p_max;
     double b2 = ddiv<FAST>(B2, W2) + vb * vb;
@@ -780,9 +825,9 @@ AFD_D bool rmhd_newton(const RmhdC2PParams &c, double &Z, double D, double tau, 
         if (fabs(f) < tol) return true;
         double eps = 1e-6 * pymax(1.0, Z);
         double fp = rmhd_f_of_Z<FAST>(c, Z + eps, D, tau, B2, SB, S2);
-        double dfdZ = (fp - f) / eps;
+        double dfdZ = fdiv(fp - f, eps);
         if (dfdZ == 0.0) return false;
-        double dZ = -f / dfdZ;
+        double dZ = fdiv(-f, dfdZ);
         if (dZ > 0.5 * Z) dZ = 0.5 * Z;
         if (dZ < -0.5 * Z) dZ = -0.5 * Z;
         Z += dZ;
@@ -814,7 +859,7 @@ AFD_D bool rmhd_recover(const RmhdC2PParams &c, double Z, const double *U, doubl
     double v2 = vx * vx + vy * vy + vz * vz;
     double vmax2 = c.v_max * c.v_max;
     if (v2 >= vmax2) {
-        double fac = c.v_max / sqrt(v2 + 1e-32);
+        double fac = fdiv(c.v_max, fsqrt(v2 + 1e-32));
         vx *= fac;
         vy *= fac;
         vz *= fac;
@@ -860,8 +905,8 @@ AFD_D void rmhd_c2p(const RmhdC2PParams &c, const double *U, double *q, C2PStats
     double vmax2 = c.v_max * c.v_max;
     double v20 = q0[1] * q0[1] + q0[2] * q0[2] + q0[3] * q0[3];
     if (v20 >= vmax2) v20 = vmax2 - 1e-14;
-    double W0 = 1.0 / sqrt(1.0 - v20);
-    double h0 = 1.0 + c.gfac * q0[4] / pymax(q0[0], SMALL);
+    double W0 = finvsqrt(1.0 - v20);
+    double h0 = 1.0 + fdiv(c.gfac * q0[4], pymax(q0[0], SMALL));
     double Z0 = pymax(q0[0] * h0 * W0 * W0, SMALL);
     double Z1 = pymax(D + tau + B2, SMALL);
     double tol = 1e-10 * pymax(1.0, tau);

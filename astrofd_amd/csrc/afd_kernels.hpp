@@ -90,7 +90,7 @@ template <typename T> struct FaceArgs {
 // WENO5 weight sum of the FP32 path (1 otherwise); below WENO_SUM_MIN the caller evaluates the
 // face again with RESCUE set (the rescaled FP32 WENO5).
 template <int RECON, typename T, bool RESCUE = false>
-AFD_D float recon_face(const double *__restrict__ b, long c, long s, int lim, double &qL, double &qR) {
+AFD_D float recon_face(const double *__restrict__ b, long c, long s, int lim, double &qL, double &qR, bool fuse3 = false) {
     constexpr bool mixed = sizeof(T) == 4;
     const double rL = mixed ? b[c - s] : 0.0, rR = mixed ? b[c] : 0.0;
     float smin = 1.0f;
@@ -117,8 +117,8 @@ AFD_D float recon_face(const double *__restrict__ b, long c, long s, int lim, do
             ppm_reconstruct<T>(lm3, lm2, lm1, l0, lp1, a, l);
             ppm_reconstruct<T>(um2, um1, u0, up1, up2, r, bb);
         } else if constexpr (!mixed) {  // WENO5: core/srhd_core.py:1183-1184
-            l = weno5_left<T>(lm3, lm2, lm1, l0, lp1);
-            r = weno5_right<T>(up2, up1, u0, um1, um2);
+            l = weno5_left<T>(lm3, lm2, lm1, l0, lp1, fuse3);
+            r = weno5_right<T>(up2, up1, u0, um1, um2, fuse3);
         } else if constexpr (RESCUE) {
             l = weno5_left_f32_rescaled(lm3, lm2, lm1, l0, lp1);
             r = weno5_left_f32_rescaled(up2, up1, u0, um1, um2);
@@ -145,7 +145,10 @@ template <int RECON, typename T, int NV>
 AFD_D void recon_face_all(const double *__restrict__ b, long n, long c, long s, int lim, double *qL, double *qR) {
     float smin = 1.0f;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) smin = fminf(smin, recon_face<RECON, T>(b + v * n, c, s, lim, qL[v], qR[v]));
+    for (int v = 0; v < NV; ++v) {
+        const bool fuse3 = NV == 9 && (v < 1 || v > 3);
+        smin = fminf(smin, recon_face<RECON, T>(b + v * n, c, s, lim, qL[v], qR[v], fuse3));
+    }
     if constexpr (RECON == 2 && sizeof(T) == 4) {
         if (__builtin_expect(!(smin >= WENO_SUM_MIN), 0)) {
             for (int v = 0; v < NV; ++v) recon_face<RECON, T, true>(b + v * n, c, s, lim, qL[v], qR[v]);
@@ -752,9 +755,9 @@ AFD_D double passive_weno_edge(double qm2, double qm1, double q0, double qp1, do
     const double IS0 = fma(c, sq((qm2 - 2.0 * qm1) + q0), 0.25 * sq(fma(3.0, q0, qm2 - 4.0 * qm1)));
     const double IS1 = fma(0.25, sq(qm1 - qp1), c * sq((qm1 - 2.0 * q0) + qp1));
     const double IS2 = fma(c, sq((q0 - 2.0 * qp1) + qp2), 0.25 * sq(fma(-4.0, qp1, 3.0 * q0) + qp2));
-    const double a0 = 0.1 / sq(eps + IS0), a1 = 0.6 / sq(eps + IS1), a2 = 0.3 / sq(eps + IS2);
-    const double s = a0 + a1 + a2;
-    return fma(a2 / s, p2, fma(a0 / s, p0, (a1 / s) * p1));
+    const double a0 = fdiv(0.1, sq(eps + IS0)), a1 = fdiv(0.6, sq(eps + IS1)), a2 = fdiv(0.3, sq(eps + IS2));
+    const Div<double> by(a0 + a1 + a2);
+    return fma(by(a2), p2, fma(by(a0), p0, by(a1) * p1));
 }
 AFD_D void passive_weno(const double *q, double &tL, double &tR) {
 #pragma clang fp contract(off)
@@ -799,7 +802,7 @@ AFD_D double passive_flux(int lim, const double *q, double vL, double vR, double
     const double fL = tL * vL, fR = tR * vR;  // hlle_scalar
     if (sL >= 0.0) return fL;
     if (sR <= 0.0) return fR;
-    return fma(sL * sR, tR - tL, fma(sR, fL, -(sL * fR))) / (sR - sL + SMALL);
+    return fdiv(fma(sL * sR, tR - tL, fma(sR, fL, -(sL * fR))), sR - sL + SMALL);
 }
 
 // ------------------------------------------------------------------ stage update + c2p

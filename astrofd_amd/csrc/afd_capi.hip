@@ -173,9 +173,10 @@ static void copy_words(afd_ctx *c, const void *src, void *dst, size_t bytes) {
 }
 
 // bytes: a multiple of 4 in both (arrays of doubles, floats and 32-bit counts).  On return the host
-// array of copy_up may be reused, that of copy_down holds the values.
-static hipError_t copy_up(afd_ctx *c, void *dev, const void *host, size_t bytes) {
-    if (bytes > PIN_BYTES || !pin_ready(c)) return xfer_h2d(dev, host, bytes, c->stream);
+// array of copy_up may be reused (wait false: once the stream has passed the copy), that of copy_down
+// holds the values.
+static hipError_t copy_up(afd_ctx *c, void *dev, const void *host, size_t bytes, bool wait = true) {
+    if (bytes > PIN_BYTES || !pin_ready(c)) return xfer_h2d(dev, host, bytes, c->stream, wait);
     if (c->pin_up_used)  // an earlier upload may still be reading it
         if (hipError_t e = hipStreamSynchronize(c->stream)) return e;
     memcpy(c->pin, host, bytes);
@@ -192,6 +193,26 @@ static hipError_t copy_down(afd_ctx *c, void *host, const void *dev, size_t byte
     if (e != hipSuccess) return e;
     c->pin_up_used = false;
     memcpy(host, c->pin + PIN_BYTES, bytes);
+    return hipSuccess;
+}
+
+// Two device arrays, the second small, with one wait (a wait and its host wake-up take 6 us).
+static hipError_t copy_down2(afd_ctx *c, void *host, const void *dev, size_t bytes, void *host2, const void *dev2,
+                             size_t bytes2) {
+    if (bytes2 > PIN_BYTES || !pin_ready(c)) {
+        hipError_t e = copy_down(c, host, dev, bytes);
+        return e == hipSuccess ? copy_down(c, host2, dev2, bytes2) : e;
+    }
+    char *pin = c->pin + PIN_BYTES;
+    const bool both = bytes + bytes2 <= PIN_BYTES;
+    copy_words(c, dev2, pin, bytes2);
+    if (both) copy_words(c, dev, pin + bytes2, bytes);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = both ? hipStreamSynchronize(c->stream) : xfer_d2h(host, dev, bytes, c->stream);
+    if (e != hipSuccess) return e;
+    c->pin_up_used = false;
+    memcpy(host2, pin, bytes2);
+    if (both) memcpy(host, pin + bytes2, bytes);
     return hipSuccess;
 }
 
@@ -1071,7 +1092,7 @@ static int batch(afd_ctx *c, int64_t n, const double *in, double *out, int32_t *
     if (int rc = scratch_get(c, 2 * slot + (iters ? (size_t)n * 4 : 0), &dev)) return rc;
     double *din = (double *)dev, *dout = (double *)(dev + slot);
     int *dit = iters ? (int *)(dev + 2 * slot) : nullptr;
-    hipError_t e = copy_up(c, din, in, bytes);
+    hipError_t e = copy_up(c, din, in, bytes, false);
     if (e == hipSuccess) {
         BatchArgs a{din,           dout,        dit,        c2p && c->stats_on ? c->stats_dev : nullptr,
                     (long)n,       c->p.physics, c->p.gamma, c->p.gamma / (c->p.gamma - 1.0),
@@ -1085,8 +1106,8 @@ static int batch(afd_ctx *c, int64_t n, const double *in, double *out, int32_t *
         }
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = copy_down(c, out, dout, bytes);
-    if (e == hipSuccess && iters) e = copy_down(c, iters, dit, (size_t)n * 4);
+    if (e == hipSuccess)
+        e = iters ? copy_down2(c, out, dout, bytes, iters, dit, (size_t)n * 4) : copy_down(c, out, dout, bytes);
     if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // nothing reads the staging after this
     scratch_done(c);
     if (e != hipSuccess) return fail(AFD_ERR_HIP, std::string("batch: ") + hipGetErrorString(e));

@@ -183,11 +183,11 @@ std::mutex g_mu;
 int g_refs = 0;
 Pool *g_pool = nullptr;  // never a static object: a process that exits with contexts open must not join
 
-hipError_t copy(bool down, void *host, void *dev, size_t bytes, hipStream_t s) {
+hipError_t copy(bool down, void *host, void *dev, size_t bytes, hipStream_t s, bool wait) {
     auto direct = [&]() {
         hipError_t e = down ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s)
                             : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+        return e == hipSuccess && wait ? hipStreamSynchronize(s) : e;
     };
     if (bytes < (down ? DOWN_MIN : UP_MIN)) return direct();
     Pool *p;
@@ -234,10 +234,10 @@ void xfer_release() {
 }
 
 hipError_t xfer_d2h(void *host, const void *dev, size_t bytes, hipStream_t s) {
-    return copy(true, host, (void *)dev, bytes, s);
+    return copy(true, host, (void *)dev, bytes, s, true);
 }
-hipError_t xfer_h2d(void *dev, const void *host, size_t bytes, hipStream_t s) {
-    return copy(false, (void *)host, dev, bytes, s);
+hipError_t xfer_h2d(void *dev, const void *host, size_t bytes, hipStream_t s, bool wait) {
+    return copy(false, (void *)host, dev, bytes, s, wait);
 }
 
 }  // namespace afd

@@ -12,8 +12,9 @@ void xfer_retain();
 void xfer_release();
 
 // Copy `bytes` between pageable host memory and device memory in stream order on `s` (a stream of the
-// current device) and wait for it: on return the host memory may be read or reused.
+// current device) and wait for it: on return the host memory may be read or reused.  wait false: the
+// host memory stays as it is until the caller has waited for the stream, so an upload need not.
 hipError_t xfer_d2h(void *host, const void *dev, size_t bytes, hipStream_t s);
-hipError_t xfer_h2d(void *dev, const void *host, size_t bytes, hipStream_t s);
+hipError_t xfer_h2d(void *dev, const void *host, size_t bytes, hipStream_t s, bool wait = true);
 
 }  // namespace afd

@@ -33,7 +33,6 @@ static int fail(int code, const std::string &msg) {
 
 constexpr int DRAW_SLOTS = 2;
 constexpr size_t SCRATCH_KEEP = size_t(256) << 20;
-constexpr size_t PIN_BYTES = size_t(512) << 10;
 
 struct afd_ctx {
     afd_params p{};
@@ -91,9 +90,9 @@ struct afd_ctx {
     // device staging of the pointwise batches, grown to the largest call (given back above SCRATCH_KEEP)
     void *scratch = nullptr;
     size_t scratch_cap = 0;
-    // pinned host memory: small arrays on their way up and down (PIN_BYTES each, from the first such
-    // copy on), the CFL speed and counts (written by the kernels), and the nozzle draws of the last
-    // DRAW_SLOTS fills (read by the kernel)
+    // pinned host memory: a block (from its first use on) of small arrays on their way up and down
+    // (PIN_BYTES each) and the CFL speed and counts (written by the kernels), and the nozzle draws of the
+    // last DRAW_SLOTS fills (read by the kernel)
     char *pin = nullptr;
     bool pin_up_used = false;
     double *host_out = nullptr;
@@ -159,10 +158,7 @@ __global__ __launch_bounds__(BLOCK) static void k_copy_words(const unsigned *src
 }
 
 static bool pin_ready(afd_ctx *c) {
-    if (!c->pin && hipHostMalloc((void **)&c->pin, 2 * PIN_BYTES, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        c->pin = nullptr;
-    }
+    if (!c->pin && (c->pin = xfer_pin_get())) c->host_out = (double *)(c->pin + 2 * PIN_BYTES);
     return c->pin != nullptr;
 }
 
@@ -396,10 +392,6 @@ extern "C" int afd_create(const afd_params *params, afd_ctx **out) {
     } while (0)
     xfer_retain();
     c->retained = true;
-    if (hipHostMalloc((void **)&c->host_out, 64, 0) != hipSuccess) {
-        afd_destroy(c);
-        return fail(AFD_ERR_NOMEM, "hipHostMalloc of the result words failed");
-    }
     size_t N = (size_t)g.ncell;
     for (int b = 0; b < 3; ++b) TRY(dalloc(c, (void **)&c->P[b], N * p.nv * 8));
     if (p.gr_orthonormal && (p.gr_metric == 1 || p.gr_metric == 2)) TRY(dalloc(c, (void **)&c->Puse, N * p.nv * 8));
@@ -475,8 +467,7 @@ extern "C" int afd_destroy(afd_ctx *c) {
         if (c->draws_ev[d]) (void)hipEventDestroy(c->draws_ev[d]);
         if (c->draws_pin[d]) (void)hipHostFree(c->draws_pin[d]);
     }
-    if (c->pin) (void)hipHostFree(c->pin);
-    if (c->host_out) (void)hipHostFree(c->host_out);
+    if (c->pin) xfer_pin_put(c->pin);  // the stream is idle
     if (c->retained) xfer_release();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1039,6 +1030,7 @@ extern "C" int afd_post_step_sources(afd_ctx *c, double dt, const afd_sources *s
 extern "C" int afd_max_char_speed(afd_ctx *c, double *amax) {
     if (!c || !amax) return fail(AFD_ERR_INVALID, "afd_max_char_speed: null argument");
     HIPCHK(hipSetDevice(c->p.device));
+    if (!pin_ready(c)) return fail(AFD_ERR_NOMEM, "no pinned memory for the result");
     const double gfac = c->p.gamma / (c->p.gamma - 1.0);
     const Grid &g = c->g;
     const SpeedBox &b = c->sbox;
@@ -1071,6 +1063,7 @@ extern "C" int afd_max_char_speed(afd_ctx *c, double *amax) {
 extern "C" int afd_count_nonfinite(afd_ctx *c, int64_t *count) {
     if (!c || !count) return fail(AFD_ERR_INVALID, "afd_count_nonfinite: null argument");
     HIPCHK(hipSetDevice(c->p.device));
+    if (!pin_ready(c)) return fail(AFD_ERR_NOMEM, "no pinned memory for the result");
     long n = c->g.ncell * c->p.nv;
     hipLaunchKernelGGL(k_count_nonfinite, dim3(c->red_blocks), dim3(BLOCK), 0, c->stream,
                        (const double *)c->P[c->cur], n, c->cnt_partial);

@@ -13,6 +13,7 @@
 #include <mutex>
 #include <new>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include <unistd.h>
@@ -181,6 +182,7 @@ struct Pool {
 
 std::mutex g_mu;
 int g_refs = 0;
+char *g_pins[2] = {};    // free pinned blocks
 Pool *g_pool = nullptr;  // never a static object: a process that exits with contexts open must not join
 
 hipError_t copy(bool down, void *host, void *dev, size_t bytes, hipStream_t s, bool wait) {
@@ -221,15 +223,50 @@ void xfer_retain() {
     ++g_refs;
 }
 
+char *xfer_pin_get() {
+    {
+        std::lock_guard<std::mutex> l(g_mu);
+        for (char *&b : g_pins)
+            if (b) {
+                char *r = b;
+                b = nullptr;
+                return r;
+            }
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, PIN_BLOCK, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return (char *)p;
+}
+
+void xfer_pin_put(char *block) {
+    {
+        std::lock_guard<std::mutex> l(g_mu);
+        for (char *&b : g_pins)
+            if (!b) {
+                b = block;
+                return;
+            }
+    }
+    (void)hipHostFree(block);
+}
+
 void xfer_release() {
     Pool *p = nullptr;
+    char *pins[2] = {};
     {
         std::lock_guard<std::mutex> l(g_mu);
         if (--g_refs == 0) {
             p = g_pool;
             g_pool = nullptr;
+            std::swap(pins[0], g_pins[0]);
+            std::swap(pins[1], g_pins[1]);
         }
     }
+    for (char *b : pins)
+        if (b) (void)hipHostFree(b);
     if (p && p->pid == getpid()) delete p;  // a forked child has no threads to join
 }
 

@@ -51,7 +51,7 @@ struct afd_ctx {
     double *Uc = nullptr;
     void *Fx = nullptr, *Fxc = nullptr, *Fy = nullptr, *Fz = nullptr, *zs = nullptr;
     double *aux[3] = {nullptr, nullptr, nullptr};
-    double *rhs_pass = nullptr, *rhs_out = nullptr;
+    double *rhs_out = nullptr;
     // nozzle
     bool noz_set = false;
     afd_nozzle noz{};
@@ -237,12 +237,14 @@ struct Timed {
             if (a && b) (void)hipEventRecord(a, c->stream);
         }
     }
-    ~Timed() {
+    void end() {
         if (c->timing_on && a && b) {
             (void)hipEventRecord(b, c->stream);
             c->marks.push_back({cat, a, b});
+            a = b = nullptr;
         }
     }
+    ~Timed() { end(); }
 };
 
 static int resolve_marks(afd_ctx *c) {
@@ -399,7 +401,7 @@ extern "C" int afd_create(const afd_params *params, afd_ctx **out) {
     TRY(dalloc(c, &c->Fx, N * nb * c->fsize));  // the flux-divergence accumulator in D-mode
     if (!c->dmode) {
         TRY(dalloc(c, &c->Fy, N * nb * c->fsize));
-        TRY(dalloc(c, &c->Fz, N * nb * c->fsize));
+        if (nb == 9) TRY(dalloc(c, &c->Fz, N * nb * c->fsize));
     }
     if (c->carried) {
         if (!c->dmode) TRY(dalloc(c, &c->Fxc, N * nb * c->fsize));
@@ -407,7 +409,6 @@ extern "C" int afd_create(const afd_params *params, afd_ctx **out) {
     }
     if (c->passive_flux) {
         for (int d = 0; d < 3; ++d) TRY(dalloc(c, (void **)&c->aux[d], N * 4 * 8));
-        TRY(dalloc(c, (void **)&c->rhs_pass, N * p.n_passive * 8));
     }
     TRY(dalloc(c, (void **)&c->amax_dev, AMAX_BYTES));
     if (hipMemset(c->amax_dev, 0, AMAX_BYTES) != hipSuccess) {  // the shell slots start at zero
@@ -735,7 +736,16 @@ static FaceLaunch face_launch(afd_ctx *c, const double *P) {
     return l;
 }
 
-static int run_faces(afd_ctx *c, const double *P, bool skip_y = false) {
+// The z faces of state P for the SRHD update (after run_faces, which rescales the velocities for GR).
+static FaceLaunch z_faces(afd_ctx *c, const double *P) {
+    FaceLaunch l = face_launch(c, c->Puse ? c->Puse : P);
+    l.dir = 2;
+    l.aux = c->passive_flux ? c->aux[2] : nullptr;
+    return l;
+}
+
+// skip: the direction whose faces the stage update evaluates itself (-1: none)
+static int run_faces(afd_ctx *c, const double *P, int skip) {
     if (c->Puse) {  // GR: the fluxes see the rescaled velocities (core/grhd_core.py:22-45)
         GrRescaleArgs r{P, c->Puse, c->g, c->p.ng, c->p.gr_x0, c->p.gr_mass, c->p.dx, c->p.dy, c->p.dz};
         Timed t(c, 4);
@@ -748,11 +758,11 @@ static int run_faces(afd_ctx *c, const double *P, bool skip_y = false) {
     // carried x speeds: z before x.  Flux divergence: the first launch writes D, so y (when
     // launched here) goes first
     const int order_carried[3] = {2, 0, 1}, order_plain[3] = {0, 1, 2}, order_div[3] = {1, 2, 0};
-    const int *order = c->dmode && !skip_y ? order_div : (c->carried ? order_carried : order_plain);
+    const int *order = c->dmode && skip != 1 ? order_div : (c->carried ? order_carried : order_plain);
     bool first = true;
     for (int n = 0; n < 3; ++n) {
         int d = order[n];
-        if (skip_y && d == 1) continue;  // the stage update evaluates the y faces itself
+        if (d == skip) continue;
         l.dfirst = first;
         first = false;
         l.dir = d;
@@ -765,28 +775,37 @@ static int run_faces(afd_ctx *c, const double *P, bool skip_y = false) {
         hipError_t e = (c->nb == 9) ? launch_face_rmhd(l, c->stream) : launch_face_srhd(l, c->stream);
         if (e != hipSuccess) return fail(AFD_ERR_HIP, std::string("face kernel: ") + hipGetErrorString(e));
     }
-    if (c->passive_flux) {
-        PassiveArgs a;
-        a.P = P;
-        for (int d = 0; d < 3; ++d) a.aux[d] = c->aux[d];
-        a.rhs = c->rhs_pass;
-        a.g = c->g;
-        a.lim = c->p.limiter_id;
-        a.np = c->p.n_passive;
-        a.po = c->p.passive_offset;
-        a.d[0] = c->p.dx;
-        a.d[1] = c->p.dy;
-        a.d[2] = c->p.dz;
-        Timed t(c, 4);
-        HIPCHK(launch_passive_rhs(a, c->nb == 9, c->p.recon_id, c->stream));
-    }
+    return AFD_OK;
+}
+
+// The passives of a stage (nst 0: their right-hand sides) into out, from the speeds and velocities the
+// stage's face kernels left in aux.
+static int run_passives(afd_ctx *c, int src, int in, double *out, int stage, int nst, double dt) {
+    PassiveArgs a;
+    a.P = c->Puse ? c->Puse : c->P[src];
+    for (int d = 0; d < 3; ++d) a.aux[d] = c->aux[d];
+    const size_t o = (size_t)c->p.passive_offset * c->g.ncell;
+    a.out = out;
+    a.P0 = c->P[in] + o;
+    a.Pin = c->P[src] + o;
+    a.stage = stage;
+    a.nst = nst;
+    a.dt = dt;
+    a.g = c->g;
+    a.lim = c->p.limiter_id;
+    a.np = c->p.n_passive;
+    a.po = c->p.passive_offset;
+    a.d[0] = c->p.dx;
+    a.d[1] = c->p.dy;
+    a.d[2] = c->p.dz;
+    Timed t(c, 4);
+    HIPCHK(launch_passives(a, c->nb == 9, c->p.recon_id, c->stream));
     return AFD_OK;
 }
 
 static UpdLaunch upd_launch(afd_ctx *c, const double *Pin, const double *P0, double *Pout, int stage, int nst,
                             double dt) {
     UpdLaunch l;
-    l.nb = c->nb;
     l.mixed = c->p.precision == AFD_PREC_MIXED;
     UpdArgs<double> &a = l.a;
     a.P0 = P0;
@@ -798,14 +817,13 @@ static UpdLaunch upd_launch(afd_ctx *c, const double *Pin, const double *P0, dou
     a.Fy = (const double *)c->Fy;
     a.Fz = (const double *)c->Fz;
     a.D = c->dmode ? (const float *)c->Fx : nullptr;
-    a.rhs_pass = c->passive_flux ? c->rhs_pass : nullptr;
     a.stats = c->stats_on ? c->stats_dev : nullptr;
     a.flags = c->stats_on ? c->flags_dev : nullptr;
     a.g = c->g;
     a.stage = stage;
     a.nst = nst;
     a.n_resist = c->nb == 9 ? c->p.n_resist : 0;
-    a.np = c->p.n_passive;
+    a.np = c->passive_flux ? 0 : c->p.n_passive;
     a.po = c->p.passive_offset;
     a.dt = dt;
     a.dx = c->p.dx;
@@ -847,18 +865,20 @@ extern "C" int afd_step(afd_ctx *c, double dt) {
     c->speed_valid = false;
     for (int s = 0; s < nst; ++s) {
         int dst = (s % 2 == 0) ? a : b;
-        int rc = run_faces(c, c->P[src], c->fused);
+        int rc = run_faces(c, c->P[src], c->nb == 5 ? 2 : (c->fused ? 1 : -1));
         if (rc) return rc;
         UpdLaunch l = upd_launch(c, c->P[src], c->P[in], c->P[dst], s, nst, dt);
         if (c->nb == 5 && s == nst - 1) {  // SRHD: the next step's CFL speed from the last stage
             HIPCHK(hipMemsetAsync(c->amax_dev, 0, AMAX_BOX_BYTES, c->stream));
             l.a.amax = c->amax_dev;
         }
-        Timed t(c, 3);
-        hipError_t e;
         if (c->repair_qcount)
             HIPCHK(hipMemsetAsync(c->repair_qcount, 0, sizeof(unsigned) * QUEUE_SLOTS, c->stream));
-        if (c->fused) {  // the y faces with the stage update
+        hipError_t e;
+        Timed t(c, 3);
+        if (c->nb == 5) {
+            e = launch_update_srhd(z_faces(c, c->P[src]), l, false, c->stream);
+        } else if (c->fused) {  // the y faces with the stage update
             FaceLaunch fl = face_launch(c, c->Puse ? c->Puse : c->P[src]);
             fl.dir = 1;
             fl.idn = (float)(1.0 / c->p.dy);
@@ -870,6 +890,11 @@ extern "C" int afd_step(afd_ctx *c, double dt) {
         if (e == hipSuccess && c->repair_queue)  // cells whose FP32 right-hand side was not finite
             e = launch_repair(face_launch(c, c->Puse ? c->Puse : c->P[src]), l, c->stream);
         if (e != hipSuccess) return fail(AFD_ERR_HIP, std::string("update kernel: ") + hipGetErrorString(e));
+        t.end();
+        if (c->passive_flux) {
+            double *out = c->P[dst] + (size_t)c->p.passive_offset * c->g.ncell;
+            if ((rc = run_passives(c, src, in, out, s, nst, dt))) return rc;
+        }
         src = dst;
     }
     c->cur = src;
@@ -884,11 +909,14 @@ extern "C" int afd_compute_rhs(afd_ctx *c, double *host, int64_t n) {
     if (n != (int64_t)nrhs * c->g.ncell) return fail(AFD_ERR_INVALID, "rhs size must be (nb + n_passive) * cells");
     HIPCHK(hipSetDevice(c->p.device));
     if (!c->rhs_out) ALLOC(c, c->rhs_out, (size_t)nrhs * c->g.ncell * 8);
-    int rc = run_faces(c, c->P[c->cur]);
+    int rc = run_faces(c, c->P[c->cur], c->nb == 5 ? 2 : -1);
     if (rc) return rc;
     UpdLaunch l = upd_launch(c, c->P[c->cur], c->P[c->cur], c->rhs_out, 0, 2, 0.0);
-    hipError_t e = launch_update(l, true, c->stream);
+    hipError_t e = c->nb == 5 ? launch_update_srhd(z_faces(c, c->P[c->cur]), l, true, c->stream)
+                              : launch_update(l, true, c->stream);
     if (e != hipSuccess) return fail(AFD_ERR_HIP, std::string("rhs kernel: ") + hipGetErrorString(e));
+    if (c->passive_flux && (rc = run_passives(c, c->cur, c->cur, c->rhs_out + (size_t)c->nb * c->g.ncell, 0, 0, 0.0)))
+        return rc;
     HIPCHK(copy_down(c, host, c->rhs_out, (size_t)n * 8));
     return AFD_OK;
 }

@@ -43,7 +43,8 @@ AFD_D void passive_dir(const PassiveArgs &a, const double *__restrict__ b, long 
     }
 }
 
-template <int MODE> __global__ __launch_bounds__(BLOCK) void k_passive_rhs(PassiveArgs a) {
+template <int MODE> __global__ __launch_bounds__(BLOCK) void k_passives(PassiveArgs a) {
+#pragma clang fp contract(off)
     const Grid &g = a.g;
     const long c = (long)blockIdx.x * BLOCK + threadIdx.x;
     if (c >= g.ncell) return;
@@ -57,15 +58,21 @@ template <int MODE> __global__ __launch_bounds__(BLOCK) void k_passive_rhs(Passi
         passive_dir<MODE, 1>(a, b, c, ijk, r);
         passive_dir<MODE, 2>(a, b, c, ijk, r);
     }
-    a.rhs[t * g.ncell + c] = r;
+    const long o = t * g.ncell + c;
+    if (a.nst == 0) {
+        a.out[o] = r;
+    } else {
+        const double dr = a.dt * r;
+        a.out[o] = ssprk_combine(a.stage, a.nst, a.P0[o], a.Pin[o], dr);
+    }
 }
 
 // physics and recon: a context with passive fluxes (RMHD MUSCL, SRHD MUSCL or PPM)
-hipError_t launch_passive_rhs(const PassiveArgs &a, bool rmhd, int recon, hipStream_t s) {
+hipError_t launch_passives(const PassiveArgs &a, bool rmhd, int recon, hipStream_t s) {
     const dim3 grid(grid1d(a.g.ncell).x, (unsigned)a.np);
-    if (rmhd) hipLaunchKernelGGL(k_passive_rhs<PASS_RMHD_MUSCL>, grid, dim3(BLOCK), 0, s, a);
-    else if (recon == 0) hipLaunchKernelGGL(k_passive_rhs<PASS_SRHD_MUSCL>, grid, dim3(BLOCK), 0, s, a);
-    else hipLaunchKernelGGL(k_passive_rhs<PASS_SRHD_PPM>, grid, dim3(BLOCK), 0, s, a);
+    if (rmhd) hipLaunchKernelGGL(k_passives<PASS_RMHD_MUSCL>, grid, dim3(BLOCK), 0, s, a);
+    else if (recon == 0) hipLaunchKernelGGL(k_passives<PASS_SRHD_MUSCL>, grid, dim3(BLOCK), 0, s, a);
+    else hipLaunchKernelGGL(k_passives<PASS_SRHD_PPM>, grid, dim3(BLOCK), 0, s, a);
     return hipGetLastError();
 }
 
@@ -458,40 +465,25 @@ hipError_t launch_face_rmhd(const FaceLaunch &l, hipStream_t s) {
 
 // One stage update: k_update (flux divergence, SSPRK, con2prim).  With a Newton start other than
 // the plain one, rejected cells are queued and solved densely by k_c2p_queue afterwards.
-template <int NB, typename F, bool LEARNED> static void upd_stage(const UpdArgs<F> &a, dim3 grid, hipStream_t s) {
-    if constexpr (NB == 9) {
-        if (a.queue) {
-            (void)hipMemsetAsync(a.qcount, 0, sizeof(unsigned) * QUEUE_SLOTS, s);
-            hipLaunchKernelGGL((k_update<NB, F, LEARNED>), grid, dim3(BLOCK), 0, s, a);
-            hipLaunchKernelGGL((k_c2p_queue<F>), dim3(16, QUEUE_SLOTS), dim3(BLOCK), 0, s, a);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((k_update<NB, F, LEARNED>), grid, dim3(BLOCK), 0, s, a);
+template <typename F, bool LEARNED> static void upd_stage(const UpdArgs<F> &a, dim3 grid, hipStream_t s) {
+    if (a.queue) (void)hipMemsetAsync(a.qcount, 0, sizeof(unsigned) * QUEUE_SLOTS, s);
+    k_update<9, F, LEARNED><<<grid, dim3(BLOCK), 0, s>>>(a);
+    if (a.queue) hipLaunchKernelGGL((k_c2p_queue<F>), dim3(16, QUEUE_SLOTS), dim3(BLOCK), 0, s, a);
 }
 
-template <int NB, typename F> static void upd(const UpdLaunch &l, bool rhs_only, hipStream_t s) {
+template <typename F> static void upd(const UpdLaunch &l, bool rhs_only, hipStream_t s) {
     UpdArgs<F> a;
     static_assert(sizeof(UpdArgs<F>) == sizeof(UpdArgs<double>), "layout");
     memcpy((void *)&a, (const void *)&l.a, sizeof(a));
     dim3 grid = grid1d(l.a.g.ncell);
-    if (rhs_only) hipLaunchKernelGGL((k_rhs<NB, F>), grid, dim3(BLOCK), 0, s, a);
-    else if constexpr (NB == 9) {
-        if (l.a.mlp) upd_stage<NB, F, true>(a, grid, s);
-        else upd_stage<NB, F, false>(a, grid, s);
-    } else {
-        upd_stage<NB, F, false>(a, grid, s);
-    }
+    if (rhs_only) hipLaunchKernelGGL((k_rhs<9, F>), grid, dim3(BLOCK), 0, s, a);
+    else if (l.a.mlp) upd_stage<F, true>(a, grid, s);
+    else upd_stage<F, false>(a, grid, s);
 }
 
 hipError_t launch_update(const UpdLaunch &l, bool rhs_only, hipStream_t s) {
-    if (l.nb == 9) {
-        if (l.mixed) upd<9, float>(l, rhs_only, s);
-        else upd<9, double>(l, rhs_only, s);
-    } else {
-        if (l.mixed) upd<5, float>(l, rhs_only, s);
-        else upd<5, double>(l, rhs_only, s);
-    }
+    if (l.mixed) upd<float>(l, rhs_only, s);
+    else upd<double>(l, rhs_only, s);
     return hipGetLastError();
 }
 

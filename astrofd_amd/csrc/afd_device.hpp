@@ -203,6 +203,20 @@ template <typename T> AFD_D T weno5_left(T qm2, T qm1, T q0, T qp1, T qp2, bool 
     T p2 = T(1.0 / 3.0) * q0 + T(5.0 / 6.0) * qp1 - T(1.0 / 6.0) * qp2;
     return w0 * p0 + w1 * p1 + w2 * p2;
 }
+// The same with the candidate polynomials' fused multiply-adds written out too, as the SRHD x and y faces
+// are compiled: the edge values of one cell evaluated together, hi = weno5_left, lo = weno5_right.
+AFD_D double weno5_edge(double qm2, double qm1, double q0, double qp1, double qp2, bool right) {
+#pragma clang fp contract(off)
+    double IS0, IS1, IS2;
+    weno5_indicators(qm2, qm1, q0, qp1, qp2, false, IS0, IS1, IS2);
+    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0, c56 = 5.0 / 6.0;
+    const double p0 = fma(11.0 / 6.0, q0, fma(c13, qm2, -((7.0 / 6.0) * qm1)));
+    const double p1 = fma(c13, qp1, fma(c56, q0, -(c16 * qm1)));
+    const double p2 = fma(-c16, qp2, right ? fma(c56, qp1, c13 * q0) : fma(c13, q0, c56 * qp1));
+    const double a0 = fdiv(0.1, sq(1e-12 + IS0)), a1 = fdiv(0.6, sq(1e-12 + IS1)), a2 = fdiv(0.3, sq(1e-12 + IS2));
+    const Div<double> by(a0 + a1 + a2);
+    return fma(by(a2), p2, fma(by(a0), p0, by(a1) * p1));
+}
 // core/srhd_core.py:361-377 (mirror image)
 template <typename T> AFD_D T weno5_right(T qp2, T qp1, T q0, T qm1, T qm2, bool fuse3) {
     return weno5_left(qp2, qp1, q0, qm1, qm2, fuse3);

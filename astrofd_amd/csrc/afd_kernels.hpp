@@ -6,6 +6,7 @@
 //       lanes along z, writes the face flux at the index of cell c;
 //   k_update: one thread per cell (ghosts included): flux differences, GLM and
 //       resistive sources, the SSPRK combination in FP64 and FP64 con2prim.
+//       SRHD (k_update_faces_z, k_update<5, float, false>): the z faces too, which have no kernel.
 // For RMHD PPM/WENO the x face of cell c is evaluated twice (Q3 of the
 // reference): with its own HLL speeds (the right face of cell c-1) and with the
 // speeds carried from the z-back face of the cell that precedes c in i->j->k order
@@ -229,23 +230,20 @@ AFD_D void diss_flux(const double *__restrict__ P, long n, long cell, const T *q
     }
 }
 
-template <int RECON, int RIEM, int DIR, typename T>
-__global__ __launch_bounds__(BLOCK) void k_face_srhd(FaceArgs<T> a) {
-    const Grid &g = a.g;
-    int i, j, k;
-    if (!face_coords<DIR>(g, a.dk, a.dn, face_thread<DIR>(), i, j, k)) return;
-    const long c = cidx(g, i, j, k), s = dstride<DIR>(g);
-    double qLd[5], qRd[5];
-    recon_face_all<RECON, T, 5>(a.P, g.ncell, c, s, a.lim, qLd, qRd);
+// The flux F of the face between cells cl and cr (= cl + the stride along DIR) from its reconstructed
+// states; aux: the speeds and velocities the passive fluxes need.
+template <int RIEM, int DIR, typename T>
+AFD_D void srhd_face(const FaceArgs<T> &a, double *qLd, double *qRd, long cl, long cr, T *F, double *aux) {
+    const long n = a.g.ncell;
     if (a.diss & 1) {  // add_pi_lr, core/srhd_core.py:394-399 (MUSCL faces, PASSIVE_OFFSET > 5)
-        qLd[4] += a.P[5 * g.ncell + c - s];
-        qRd[4] += a.P[5 * g.ncell + c];
+        qLd[4] += a.P[5 * n + cl];
+        qRd[4] += a.P[5 * n + cr];
     }
     srhd_floor(a.p_max, a.v_max, qLd);
     srhd_floor(a.p_max, a.v_max, qRd);
     T WL = (T)lorentz_guarded<sizeof(T) == 4>(qLd[1] * qLd[1] + qLd[2] * qLd[2] + qLd[3] * qLd[3]);
     T WR = (T)lorentz_guarded<sizeof(T) == 4>(qRd[1] * qRd[1] + qRd[2] * qRd[2] + qRd[3] * qRd[3]);
-    T qL[5], qR[5], UL[5], UR[5], FL[5], FR[5], F[5];
+    T qL[5], qR[5], UL[5], UR[5], FL[5], FR[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
         qL[v] = (T)qLd[v];
@@ -256,8 +254,8 @@ __global__ __launch_bounds__(BLOCK) void k_face_srhd(FaceArgs<T> a) {
     srhd_flux<DIR>(qL, UL, FL);
     srhd_flux<DIR>(qR, UR, FR);
     for (int r = 0; r < (a.diss >> 1); ++r) {  // apply_diss_flux: once per MUSCL face, twice per PPM face
-        diss_flux<DIR>(a.P, g.ncell, c - s, qL, FL);
-        diss_flux<DIR>(a.P, g.ncell, c, qR, FR);
+        diss_flux<DIR>(a.P, n, cl, qL, FL);
+        diss_flux<DIR>(a.P, n, cr, qR, FR);
     }
     T csL = srhd_sound_speed(a.ph, qL[0], qL[4]), csR = srhd_sound_speed(a.ph, qR[0], qR[4]);
     T lmL, lpL, lmR, lpR;
@@ -268,13 +266,73 @@ __global__ __launch_bounds__(BLOCK) void k_face_srhd(FaceArgs<T> a) {
         hllc5<1 + DIR>(UL, UR, FL, FR, sL, sR, qL[4], qR[4], qL[1 + DIR], qR[1 + DIR], F);
     else
         hlle_vec<5>(UL, UR, FL, FR, sL, sR, F);
+    if (aux) {
+        aux[cr] = sL;
+        aux[n + cr] = sR;
+        aux[2 * n + cr] = qL[1 + DIR];
+        aux[3 * n + cr] = qR[1 + DIR];
+    }
+}
+
+template <int RECON, int RIEM, int DIR, typename T>
+__global__ __launch_bounds__(BLOCK) void k_face_srhd(FaceArgs<T> a) {
+    const Grid &g = a.g;
+    int i, j, k;
+    if (!face_coords<DIR>(g, a.dk, a.dn, face_thread<DIR>(), i, j, k)) return;
+    const long c = cidx(g, i, j, k), s = dstride<DIR>(g);
+    double qLd[5], qRd[5];
+    recon_face_all<RECON, T, 5>(a.P, g.ncell, c, s, a.lim, qLd, qRd);
+    T F[5];
+    srhd_face<RIEM, DIR, T>(a, qLd, qRd, c - s, c, F, a.aux);
 #pragma unroll
     for (int v = 0; v < 5; ++v) a.F[v * g.ncell + c] = F[v];
-    if (a.aux) {
-        a.aux[c] = sL;
-        a.aux[g.ncell + c] = sR;
-        a.aux[2 * g.ncell + c] = qL[1 + DIR];
-        a.aux[3 * g.ncell + c] = qR[1 + DIR];
+}
+
+// Both edges of the cell at b along z: lo at the face with the cell below, hi at the face with the cell
+// above, the values recon_face gives the faces there (rescue, sum: as there).
+template <int RECON, typename T, bool RESCUE = false>
+AFD_D float cell_edges_z(const double *__restrict__ b, int lim, double &lo, double &hi) {
+    constexpr bool mixed = sizeof(T) == 4;
+    const double r = mixed ? b[0] : 0.0;
+    const T q0 = (T)(b[0] - r), qm1 = (T)(b[-1] - r), qp1 = (T)(b[1] - r);
+    float smin = 1.0f;
+    T l, h;
+    if constexpr (RECON == 0) {
+        const T sl = limiter<T>(lim, q0 - qm1, qp1 - q0);
+        h = q0 + T(0.5) * sl;
+        l = q0 - T(0.5) * sl;
+    } else {
+        const T qm2 = (T)(b[-2] - r), qp2 = (T)(b[2] - r);
+        if constexpr (RECON == 1) {
+            ppm_reconstruct<T>(qm2, qm1, q0, qp1, qp2, l, h);
+        } else if constexpr (!mixed) {
+            h = weno5_edge(qm2, qm1, q0, qp1, qp2, false);
+            l = weno5_edge(qp2, qp1, q0, qm1, qm2, true);
+        } else if constexpr (RESCUE) {
+            h = weno5_left_f32_rescaled(qm2, qm1, q0, qp1, qp2);
+            l = weno5_left_f32_rescaled(qp2, qp1, q0, qm1, qm2);
+        } else {
+            float s1, s2;
+            h = weno5_left_f32_eps(qm2, qm1, q0, qp1, qp2, 1e-12f, s1);
+            l = weno5_left_f32_eps(qp2, qp1, q0, qm1, qm2, 1e-12f, s2);
+            smin = fminf(s1, s2);
+        }
+    }
+    lo = mixed ? r + (double)l : (double)l;
+    hi = mixed ? r + (double)h : (double)h;
+    return smin;
+}
+
+template <int RECON, typename T>
+AFD_D void srhd_edges_z(const FaceArgs<T> &a, long c, double *lo, double *hi) {
+    const long n = a.g.ncell;
+    float smin = 1.0f;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) smin = fminf(smin, cell_edges_z<RECON, T>(a.P + v * n + c, a.lim, lo[v], hi[v]));
+    if constexpr (RECON == 2 && sizeof(T) == 4) {
+        if (__builtin_expect(!(smin >= WENO_SUM_MIN), 0)) {
+            for (int v = 0; v < 5; ++v) cell_edges_z<RECON, T, true>(a.P + v * n + c, a.lim, lo[v], hi[v]);
+        }
     }
 }
 
@@ -717,7 +775,7 @@ void k_face_rmhd_weno_march(FaceArgs<float> a) {
 // Passive fluxes of the reference's MUSCL (SRHD, RMHD) and PPM (SRHD) right-hand sides:
 // the face states of the WENO, PPM and MUSCL variants are recomputed here and combined with
 // the speeds/velocities the face kernels stored, in the reference's order of subtraction.
-// One thread per cell and passive (blockIdx.y), the scheme at compile time (k_passive_rhs<MODE>): the
+// One thread per cell and passive (blockIdx.y), the scheme at compile time (k_passives<MODE>): the
 // seven values along an axis serve both faces and every variant, and the passives of a cell run side
 // by side.  (One thread walking all passives, each face and variant gathering its own six values with
 // a wrap test on each axis: 137 us for six passives on 64 x 60 x 66, now 48; one RMHD passive on
@@ -725,7 +783,10 @@ void k_face_rmhd_weno_march(FaceArgs<float> a) {
 struct PassiveArgs {
     const double *P;
     const double *aux[3];   // per direction (sL, sR, vL, vR) x ncell
-    double *rhs;            // n_passive x ncell, zero outside the range
+    double *out;            // n_passive x ncell: the stage's new passives, or (nst 0) their right-hand sides
+    const double *P0, *Pin; // the passives of the step's and of the stage's input (SSPRK combination)
+    int stage, nst;
+    double dt;
     Grid g;
     int lim, np, po;
     double d[3];
@@ -819,11 +880,10 @@ template <typename F> struct UpdArgs {
     double *Uc;           // conserved: running stage value (FP64); the step start's is p2c(P0)
     const F *Fx, *FxL, *Fy, *Fz;  // face fluxes; FxL is the left-face x flux (carried speeds)
     const float *D;               // or (mixed RMHD WENO5 with shared edges) the FP32 flux divergence
-    const double *rhs_pass;       // passive rhs (or null = 0)
     unsigned long long *stats;    // [hydro_iters, newton_evals, fallback, bisection, invalid, learned] or null
     unsigned char *flags;         // with stats: the last stage's con2prim branch bits per cell (C2PStats::flags)
     Grid g;
-    int stage, nst, n_resist, np, po;
+    int stage, nst, n_resist, np, po;  // np 0 where k_passives updates the passives
     double dt, dx, dy, dz, glm_cp2, resistivity;
     double gamma, gfac, p_max, v_max;
     const void *mlp;              // learned-guess weights (null: plain con2prim)
@@ -1006,30 +1066,40 @@ template <int NB, typename F> AFD_D void cell_rhs_glm_resist(const UpdArgs<F> &a
     }
 }
 
+// rhs -= (Fr - Fl) / d.  FP64: the reference's division; mixed path (FP32 fluxes): times 1 / d.
+template <typename F> struct FluxDiff;
+template <> struct FluxDiff<double> {
+    Div<double> by;
+    AFD_D explicit FluxDiff(double d) : by(d) {}
+    AFD_D void operator()(double &rhs, double Fr, double Fl) const {
+#pragma clang fp contract(off)
+        rhs -= by(Fr - Fl);
+    }
+};
+template <> struct FluxDiff<float> {
+    double inv;
+    AFD_D explicit FluxDiff(double d) : inv(1.0 / d) {}
+    AFD_D void operator()(double &rhs, float Fr, float Fl) const {
+#pragma clang fp contract(off)
+        rhs -= ((double)Fr - (double)Fl) * inv;
+    }
+};
+
 // The flat RHS of a cell in the flux ranges: flux divergence, GLM and resistive sources.
 template <int NB, typename F> AFD_D void cell_rhs_flat(const UpdArgs<F> &a, long c, double *rhs) {
 #pragma clang fp contract(off)
     const Grid &g = a.g;
-    if constexpr (sizeof(F) == 8) {  // FP64 path: the reference's divisions
-        const Div<double> bx(a.dx), by(a.dy), bz(a.dz);
-#pragma unroll
-        for (int v = 0; v < NB; ++v) {
-            long o = v * g.ncell + c;
-            rhs[v] -= bx((double)a.Fx[o + g.sx] - (double)a.FxL[o]);
-            rhs[v] -= by((double)a.Fy[o + g.sy] - (double)a.Fy[o]);
-            rhs[v] -= bz((double)a.Fz[o + 1] - (double)a.Fz[o]);
-        }
-    } else if (a.D) {  // the face kernels accumulated the divergence, already over the spacings
+    if (sizeof(F) == 4 && a.D) {  // the face kernels accumulated the divergence, already over the spacings
 #pragma unroll
         for (int v = 0; v < NB; ++v) rhs[v] -= (double)a.D[v * g.ncell + c];
-    } else {  // mixed path (FP32 fluxes): multiply by the inverse spacings
-        const double ix = 1.0 / a.dx, iy = 1.0 / a.dy, iz = 1.0 / a.dz;
+    } else {
+        const FluxDiff<F> x(a.dx), y(a.dy), z(a.dz);
 #pragma unroll
         for (int v = 0; v < NB; ++v) {
-            long o = v * g.ncell + c;
-            rhs[v] -= ((double)a.Fx[o + g.sx] - (double)a.FxL[o]) * ix;
-            rhs[v] -= ((double)a.Fy[o + g.sy] - (double)a.Fy[o]) * iy;
-            rhs[v] -= ((double)a.Fz[o + 1] - (double)a.Fz[o]) * iz;
+            const long o = v * g.ncell + c;
+            x(rhs[v], a.Fx[o + g.sx], a.FxL[o]);
+            y(rhs[v], a.Fy[o + g.sy], a.Fy[o]);
+            z(rhs[v], a.Fz[o + 1], a.Fz[o]);
         }
     }
     cell_rhs_glm_resist<NB, F>(a, c, rhs);
@@ -1060,7 +1130,7 @@ __global__ __launch_bounds__(BLOCK) void k_rhs(UpdArgs<F> a) {
     cell_rhs<NB, F>(a, c, in_range(g, c), rhs);
 #pragma unroll
     for (int v = 0; v < NB; ++v) a.Pout[v * g.ncell + c] = rhs[v];
-    for (int t = 0; t < a.np; ++t) a.Pout[(NB + t) * g.ncell + c] = a.rhs_pass ? a.rhs_pass[t * g.ncell + c] : 0.0;
+    for (int t = 0; t < a.np; ++t) a.Pout[(NB + t) * g.ncell + c] = 0.0;
 }
 
 // Z = rho h W^2 of a primitive state (the previous-state Newton start)
@@ -1183,13 +1253,7 @@ AFD_D void cell_update(const UpdArgs<F> &a, long c, bool live, const double *rhs
         for (int v = NB; v < a.po; ++v) a.Pout[(long)v * g.ncell + c] = a.Pin[(long)v * g.ncell + c];
         for (int t = 0; t < a.np; ++t) {
             long o = (long)(a.po + t) * g.ncell + c;
-            double rt = a.rhs_pass ? a.rhs_pass[t * g.ncell + c] : 0.0;
-            double r;
-            {
-#pragma clang fp contract(off)
-                r = a.dt * rt;
-            }
-            a.Pout[o] = ssprk_combine(a.stage, a.nst, a.P0[o], a.Pin[o], r);
+            a.Pout[o] = ssprk_combine(a.stage, a.nst, a.P0[o], a.Pin[o], 0.0);
         }
     }
     if (a.stats) wave_add_stats(a.stats, st);
@@ -1245,6 +1309,82 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(LEARNED ?
         if (live) cell_rhs<NB, F>(a, c, in_range(g, c), rhs);
         cell_update<NB, F, false>(a, c, live, rhs);
     }
+}
+
+// The SRHD stage update with the z faces in it: one lane per cell of the whole array in memory order,
+// which evaluates the cell's two z edges and the face on its low side (the other cell's edge from the
+// lane below), takes the flux on the high side from the lane above and updates the cell.  Consecutive
+// waves overlap by two cells (lanes 1..62 update).  The update is bound by HBM traffic and the faces by
+// vector instructions, so a z kernel of its own costs its time, each cell's slopes twice, and the flux
+// written and read.  256^3 FP64 HLLC:
+// 476 us of z faces and 870 of update before, 948 now; 128^3 HLLE: 28 + 61, now 60; 181 x 127 x 143
+// mixed: 50 + 140, now 165.  recon and riem as FaceLaunch's, the same for the whole launch;
+// rhs_only: the right-hand side into Pout, (5 + np) x ncell.
+constexpr int ZCELLS = 62;  // cells a wave updates
+template <typename F>
+AFD_D void update_faces_z(const FaceArgs<F> &fa, const UpdArgs<F> &ua, int recon, int riem, bool rhs_only) {
+    const Grid &g = ua.g;
+    const int lane = threadIdx.x & 63;
+    const long n = g.ncell, c = (long)(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * ZCELLS + lane - 1;
+    const bool live = lane >= 1 && lane <= ZCELLS && c < n;
+    int i = 0, j = 0, k = 0;
+    if (c >= 0 && c < n) cell_ijk(g, c, i, j, k);
+    const bool line = i >= g.r0[0] && i < g.r1[0] && j >= g.r0[1] && j < g.r1[1];
+    const bool edges = line && k >= g.r0[2] - 1 && k <= g.r1[2];  // a cell beside a face
+    const bool in = line && k >= g.r0[2] && k < g.r1[2];
+    F Fl[5], Fh[5];
+    if (__any(edges)) {
+        // lanes without a face repeat a cell that has one and store nothing
+        const long ce = edges ? c : cidx(g, g.r0[0], g.r0[1], g.r0[2]);
+        double lo[5], hi[5], L[5];
+        if (recon == 0) srhd_edges_z<0, F>(fa, ce, lo, hi);
+        else if (recon == 1) srhd_edges_z<1, F>(fa, ce, lo, hi);
+        else srhd_edges_z<2, F>(fa, ce, lo, hi);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) L[v] = __shfl_up(hi[v], 1);
+        const bool face = live && line && k >= g.r0[2] && k <= g.r1[2];
+        double *aux = face ? fa.aux : nullptr;
+        if (riem == 1) srhd_face<1, 2, F>(fa, L, lo, ce - 1, ce, Fl, aux);
+        else srhd_face<0, 2, F>(fa, L, lo, ce - 1, ce, Fl, aux);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) Fh[v] = __shfl_down(Fl[v], 1);
+    }
+    double rhs[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (live) {
+        if (in) {
+            const FluxDiff<F> x(ua.dx), y(ua.dy), z(ua.dz);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+                const long o = v * n + c;
+                x(rhs[v], ua.Fx[o + g.sx], ua.Fx[o]);
+                y(rhs[v], ua.Fy[o + g.sy], ua.Fy[o]);
+                z(rhs[v], Fh[v], Fl[v]);
+            }
+        }
+        if (ua.gr) gr_source<5, F>(ua, c, rhs);
+    }
+    if (!rhs_only) {
+        cell_update<5, F, false>(ua, c, live, rhs);
+    } else if (live) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) ua.Pout[v * n + c] = rhs[v];
+        for (int t = 0; t < ua.np; ++t) ua.Pout[(5 + t) * n + c] = 0.0;
+    }
+}
+
+// FP64: the scheme at compile time (all of them in one kernel: 108 registers and 4 waves a SIMD, 1026 us
+// where MUSCL's own takes 90, 5 waves and 948 us; held to 5 it spills and 128^3 takes 80 us for 60).
+// Mixed: one kernel for every scheme (86 registers, 5 waves).
+template <int RECON, int RIEM>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_update_faces_z(
+    FaceArgs<double> fa, UpdArgs<double> ua, bool rhs_only) {
+    update_faces_z<double>(fa, ua, RECON, RIEM, rhs_only);
+}
+template <int NB, typename F, bool LEARNED>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_update(
+    FaceArgs<F> fa, UpdArgs<F> ua, int recon, int riem, bool rhs_only) {
+    static_assert(NB == 5 && sizeof(F) == 4 && !LEARNED, "mixed SRHD");
+    update_faces_z<F>(fa, ua, recon, riem, rhs_only);
 }
 
 // y pencils fused with the stage update (mixed RMHD WENO5 on the flux-divergence path): the pencil

@@ -55,16 +55,19 @@ inline long face_count(const Grid &g, int dir) {
 hipError_t launch_face_srhd(const FaceLaunch &l, hipStream_t s);
 hipError_t launch_face_rmhd(const FaceLaunch &l, hipStream_t s);
 
-// Stage update / rhs-only launch.  flux pointers typed by `mixed`.
+// RMHD stage update / rhs-only launch.  flux pointers typed by `mixed`.
 struct UpdLaunch {
     UpdArgs<double> a;  // flux pointers reinterpreted as float when mixed
     bool mixed;
-    int nb;
 };
 hipError_t launch_update(const UpdLaunch &l, bool rhs_only, hipStream_t s);
 
-// Passive right-hand sides into a.rhs (contexts with passive fluxes: RMHD MUSCL, SRHD MUSCL and PPM).
-hipError_t launch_passive_rhs(const PassiveArgs &a, bool rmhd, int recon, hipStream_t s);
+// SRHD: the stage update with the z faces in it (l: the z faces), or with rhs_only the right-hand side
+// into u.a.Pout.
+hipError_t launch_update_srhd(const FaceLaunch &l, const UpdLaunch &u, bool rhs_only, hipStream_t s);
+
+// The passives of a stage into a.out (contexts with passive fluxes: RMHD MUSCL, SRHD MUSCL and PPM).
+hipError_t launch_passives(const PassiveArgs &a, bool rmhd, int recon, hipStream_t s);
 
 // Mixed RMHD WENO5 on the flux-divergence path: the y faces fused with the stage update
 // (k_face_march_update), the ghost shell's update and the learned start's fallback queue.

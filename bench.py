@@ -282,6 +282,8 @@ def kernel_name(s, which, mixed, learned, face_path=0):
     if which == "stage_update_c2p":
         if v == 4:
             return f"k_face_march_update<{rid}, {'true' if learned else 'false'}>"
+        if nb == 5 and not mixed:  # SRHD updates evaluate the z faces; FP64: the scheme at compile time
+            return f"k_update_faces_z<{recon_id(s['RECON'])}, {rid}>"
         return f"k_update<{nb}, {T}, {'true' if learned else 'false'}>"
     d = {"face_x": 0, "face_y": 1, "face_z": 2}[which]
     if v >= 3:
@@ -311,13 +313,14 @@ def impl_update_bytes(s, mixed, face_path=0):
     """HBM bytes per cell of one stage update as this implementation moves them, averaged over the
     stages: read P0 (U0 = p2c(P0) every stage), read U_s-1 (stages > 0), write U_s (not the last
     stage), write P_s, read psi and the passives of P_s-1, and the face terms: one FP32 flux
-    divergence on the flux-divergence path, else one read of each face-flux array."""
+    divergence on the flux-divergence path, else one read of each face-flux array (SRHD: of the x and y
+    fluxes, and of P_s-1 for the z faces, which the update evaluates)."""
     nb = 9 if s["PHYSICS"] == "rmhd" else 5
     nv = nvars(s)
     nst = 3 if s["RK_ORDER"] == 3 else 2
     fb = 4 if mixed else 8
     carried = nb == 9 and s["RECON"] != "muscl"
-    face = nb * 4 if flux_divergence_path(s, mixed, face_path) else (4 if carried else 3) * nb * fb
+    face = 2 * nb * fb + nb * 8 if nb == 5 else nb * 4 if flux_divergence_path(s, mixed, face_path) else (4 if carried else 3) * nb * fb
     per = []
     for st in range(nst):
         b = nv * 8 + nv * 8 + face + (8 if nb == 9 else 0) + (nv - nb) * 8

@@ -156,6 +156,22 @@ template <typename T> AFD_D T limiter(int lid, T dqL, T dqR) {
     return minmod(T(0.5) * (dqL + dqR), T(2) * mm);
 }
 
+// The limited slopes of N pairs of differences.  The limiter is chosen once for all of them: a choice
+// per slope splits the code into blocks that the loads of the next slopes do not cross, so that the
+// variables' loads wait for one another.
+template <int N, typename T> AFD_D void limiters(int lid, const T *dqL, const T *dqR, T *sl) {
+    if (lid == 1) {
+#pragma unroll
+        for (int m = 0; m < N; ++m) sl[m] = limiter<T>(1, dqL[m], dqR[m]);
+    } else if (lid == 2) {
+#pragma unroll
+        for (int m = 0; m < N; ++m) sl[m] = limiter<T>(2, dqL[m], dqR[m]);
+    } else {
+#pragma unroll
+        for (int m = 0; m < N; ++m) sl[m] = limiter<T>(0, dqL[m], dqR[m]);
+    }
+}
+
 // core/srhd_core.py:327-341
 template <typename T> AFD_D void ppm_reconstruct(T qm2, T qm1, T q0, T qp1, T qp2, T &oL, T &oR) {
     T qL = T(7.0 / 12.0) * (qm1 + q0) - T(1.0 / 12.0) * (qm2 + qp1);

@@ -140,10 +140,46 @@ AFD_D float recon_face(const double *__restrict__ b, long c, long s, int lim, do
     return smin;
 }
 
+// The SRHD MUSCL states (core/srhd_core.py:486-533) with every load before the first slope: recon_face
+// chooses the limiter for each slope, and the blocks that makes keep the loads of the next variable
+// behind it, five round trips one after another (faces of 256^3 in FP64: 478 and 475 -> 459 and 455 us,
+// 128^3: 33 and 29 -> 30 and 27; update_faces_z there 948 -> 919, 60 -> 58).
+template <typename T, int NV>
+AFD_D void muscl_face_all(const double *__restrict__ b, long n, long c, long s, int lim, double *qL, double *qR) {
+    constexpr bool mixed = sizeof(T) == 4;
+    double bm1[NV], b0[NV];
+    T dl[2 * NV], dr[2 * NV], q[2 * NV], sl[2 * NV];  // left states (cell c - s), then right ones (cell c)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const double *f = b + v * n;
+        const double bm2 = f[c - 2 * s], bp1 = f[c + s];
+        bm1[v] = f[c - s];
+        b0[v] = f[c];
+        const double rL = mixed ? bm1[v] : 0.0, rR = mixed ? b0[v] : 0.0;
+        q[v] = (T)(bm1[v] - rL);
+        dl[v] = q[v] - (T)(bm2 - rL);
+        dr[v] = (T)(b0[v] - rL) - q[v];
+        q[NV + v] = (T)(b0[v] - rR);
+        dl[NV + v] = q[NV + v] - (T)(bm1[v] - rR);
+        dr[NV + v] = (T)(bp1 - rR) - q[NV + v];
+    }
+    limiters<2 * NV, T>(lim, dl, dr, sl);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const T l = q[v] + T(0.5) * sl[v], r = q[NV + v] - T(0.5) * sl[NV + v];
+        qL[v] = mixed ? bm1[v] + (double)l : (double)l;
+        qR[v] = mixed ? b0[v] + (double)r : (double)r;
+    }
+}
+
 // The face states of NV variables (fields at b + v * n); the FP32 WENO5 lanes whose weights
 // underflow evaluate again with the rescaled WENO5.
 template <int RECON, typename T, int NV>
 AFD_D void recon_face_all(const double *__restrict__ b, long n, long c, long s, int lim, double *qL, double *qR) {
+    if constexpr (RECON == 0 && NV == 5) {
+        muscl_face_all<T, NV>(b, n, c, s, lim, qL, qR);
+        return;
+    }
     float smin = 1.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
@@ -291,32 +327,26 @@ __global__ __launch_bounds__(BLOCK) void k_face_srhd(FaceArgs<T> a) {
 // Both edges of the cell at b along z: lo at the face with the cell below, hi at the face with the cell
 // above, the values recon_face gives the faces there (rescue, sum: as there).
 template <int RECON, typename T, bool RESCUE = false>
-AFD_D float cell_edges_z(const double *__restrict__ b, int lim, double &lo, double &hi) {
+AFD_D float cell_edges_z(const double *__restrict__ b, double &lo, double &hi) {
     constexpr bool mixed = sizeof(T) == 4;
     const double r = mixed ? b[0] : 0.0;
     const T q0 = (T)(b[0] - r), qm1 = (T)(b[-1] - r), qp1 = (T)(b[1] - r);
     float smin = 1.0f;
     T l, h;
-    if constexpr (RECON == 0) {
-        const T sl = limiter<T>(lim, q0 - qm1, qp1 - q0);
-        h = q0 + T(0.5) * sl;
-        l = q0 - T(0.5) * sl;
+    const T qm2 = (T)(b[-2] - r), qp2 = (T)(b[2] - r);
+    if constexpr (RECON == 1) {
+        ppm_reconstruct<T>(qm2, qm1, q0, qp1, qp2, l, h);
+    } else if constexpr (!mixed) {
+        h = weno5_edge(qm2, qm1, q0, qp1, qp2, false);
+        l = weno5_edge(qp2, qp1, q0, qm1, qm2, true);
+    } else if constexpr (RESCUE) {
+        h = weno5_left_f32_rescaled(qm2, qm1, q0, qp1, qp2);
+        l = weno5_left_f32_rescaled(qp2, qp1, q0, qm1, qm2);
     } else {
-        const T qm2 = (T)(b[-2] - r), qp2 = (T)(b[2] - r);
-        if constexpr (RECON == 1) {
-            ppm_reconstruct<T>(qm2, qm1, q0, qp1, qp2, l, h);
-        } else if constexpr (!mixed) {
-            h = weno5_edge(qm2, qm1, q0, qp1, qp2, false);
-            l = weno5_edge(qp2, qp1, q0, qm1, qm2, true);
-        } else if constexpr (RESCUE) {
-            h = weno5_left_f32_rescaled(qm2, qm1, q0, qp1, qp2);
-            l = weno5_left_f32_rescaled(qp2, qp1, q0, qm1, qm2);
-        } else {
-            float s1, s2;
-            h = weno5_left_f32_eps(qm2, qm1, q0, qp1, qp2, 1e-12f, s1);
-            l = weno5_left_f32_eps(qp2, qp1, q0, qm1, qm2, 1e-12f, s2);
-            smin = fminf(s1, s2);
-        }
+        float s1, s2;
+        h = weno5_left_f32_eps(qm2, qm1, q0, qp1, qp2, 1e-12f, s1);
+        l = weno5_left_f32_eps(qp2, qp1, q0, qm1, qm2, 1e-12f, s2);
+        smin = fminf(s1, s2);
     }
     lo = mixed ? r + (double)l : (double)l;
     hi = mixed ? r + (double)h : (double)h;
@@ -326,12 +356,33 @@ AFD_D float cell_edges_z(const double *__restrict__ b, int lim, double &lo, doub
 template <int RECON, typename T>
 AFD_D void srhd_edges_z(const FaceArgs<T> &a, long c, double *lo, double *hi) {
     const long n = a.g.ncell;
+    if constexpr (RECON == 0) {
+        double b0[5];
+        T q[5], dl[5], dr[5], sl[5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            const double *b = a.P + v * n + c;
+            b0[v] = b[0];
+            const double r = sizeof(T) == 4 ? b0[v] : 0.0;
+            q[v] = (T)(b0[v] - r);
+            dl[v] = q[v] - (T)(b[-1] - r);
+            dr[v] = (T)(b[1] - r) - q[v];
+        }
+        limiters<5, T>(a.lim, dl, dr, sl);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            const T h = q[v] + T(0.5) * sl[v], l = q[v] - T(0.5) * sl[v];
+            hi[v] = sizeof(T) == 4 ? b0[v] + (double)h : (double)h;
+            lo[v] = sizeof(T) == 4 ? b0[v] + (double)l : (double)l;
+        }
+        return;
+    }
     float smin = 1.0f;
 #pragma unroll
-    for (int v = 0; v < 5; ++v) smin = fminf(smin, cell_edges_z<RECON, T>(a.P + v * n + c, a.lim, lo[v], hi[v]));
+    for (int v = 0; v < 5; ++v) smin = fminf(smin, cell_edges_z<RECON, T>(a.P + v * n + c, lo[v], hi[v]));
     if constexpr (RECON == 2 && sizeof(T) == 4) {
         if (__builtin_expect(!(smin >= WENO_SUM_MIN), 0)) {
-            for (int v = 0; v < 5; ++v) cell_edges_z<RECON, T, true>(a.P + v * n + c, a.lim, lo[v], hi[v]);
+            for (int v = 0; v < 5; ++v) cell_edges_z<RECON, T, true>(a.P + v * n + c, lo[v], hi[v]);
         }
     }
 }

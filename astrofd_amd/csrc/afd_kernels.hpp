@@ -353,28 +353,40 @@ AFD_D float cell_edges_z(const double *__restrict__ b, double &lo, double &hi) {
     return smin;
 }
 
+// Both MUSCL edges of a cell from its five base variables q0 and those before (qm) and after it (qp)
+template <typename T>
+AFD_D void muscl_edges(int lim, const double *qm, const double *q0, const double *qp, double *lo, double *hi) {
+    constexpr bool mixed = sizeof(T) == 4;
+    T q[5], dl[5], dr[5], sl[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const double r = mixed ? q0[v] : 0.0;
+        q[v] = (T)(q0[v] - r);
+        dl[v] = q[v] - (T)(qm[v] - r);
+        dr[v] = (T)(qp[v] - r) - q[v];
+    }
+    limiters<5, T>(lim, dl, dr, sl);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const T h = q[v] + T(0.5) * sl[v], l = q[v] - T(0.5) * sl[v];
+        hi[v] = mixed ? q0[v] + (double)h : (double)h;
+        lo[v] = mixed ? q0[v] + (double)l : (double)l;
+    }
+}
+
 template <int RECON, typename T>
 AFD_D void srhd_edges_z(const FaceArgs<T> &a, long c, double *lo, double *hi) {
     const long n = a.g.ncell;
     if constexpr (RECON == 0) {
-        double b0[5];
-        T q[5], dl[5], dr[5], sl[5];
+        double qm[5], q0[5], qp[5];
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
             const double *b = a.P + v * n + c;
-            b0[v] = b[0];
-            const double r = sizeof(T) == 4 ? b0[v] : 0.0;
-            q[v] = (T)(b0[v] - r);
-            dl[v] = q[v] - (T)(b[-1] - r);
-            dr[v] = (T)(b[1] - r) - q[v];
+            qm[v] = b[-1];
+            q0[v] = b[0];
+            qp[v] = b[1];
         }
-        limiters<5, T>(a.lim, dl, dr, sl);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            const T h = q[v] + T(0.5) * sl[v], l = q[v] - T(0.5) * sl[v];
-            hi[v] = sizeof(T) == 4 ? b0[v] + (double)h : (double)h;
-            lo[v] = sizeof(T) == 4 ? b0[v] + (double)l : (double)l;
-        }
+        muscl_edges<T>(a.lim, qm, q0, qp, lo, hi);
         return;
     }
     float smin = 1.0f;
@@ -384,6 +396,59 @@ AFD_D void srhd_edges_z(const FaceArgs<T> &a, long c, double *lo, double *hi) {
         if (__builtin_expect(!(smin >= WENO_SUM_MIN), 0)) {
             for (int v = 0; v < 5; ++v) cell_edges_z<RECON, T, true>(a.P + v * n + c, lo[v], hi[v]);
         }
+    }
+}
+
+// The x and y MUSCL faces of a large grid: a lane marches `run` faces along the normal, lanes over the
+// positions across it (z fastest).  A cell's two edges are evaluated together and the high one kept for the
+// next face, so each slope once and not twice; the cells stay in registers and the run's next one is
+// loaded while a face is worked on: 5 loads a face instead of 20, none of them waited for.  The registers
+// (128, mixed 92) leave four waves a SIMD, so it pays where runs fill the chip: FP64 256^3 459 and 455 -> 397 and
+// 413 us, mixed 181 x 127 x 143 68 and 57 -> 58 and 56, but 128^3 30 and 27 -> 31 and 31 (and PPM and
+// WENO5, whose cells do not fit the registers too, 2 to 8 % slower by runs).  a.dn divides by the
+// workgroups of one run.
+template <int RECON, int RIEM, int DIR, typename T>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 5)))
+void k_face_srhd(FaceArgs<T> a, int run) {
+    static_assert(RECON == 0 && DIR < 2, "MUSCL x and y faces");
+    constexpr int O = DIR == 0 ? 1 : 0;
+    const Grid &g = a.g;
+    const long n = g.ncell, s = dstride<DIR>(g);
+    const unsigned nk = g.r1[2] - g.r0[2], npos = nk * (unsigned)(g.r1[O] - g.r0[O]);
+    const unsigned b = (unsigned)xcd_chunked_block(blockIdx.x, gridDim.x), r = udiv(a.dn, b);
+    const unsigned pos = (b - r * ((npos + BLOCK - 1) / BLOCK)) * BLOCK + threadIdx.x;
+    if (pos >= npos) return;
+    const unsigned row = udiv(a.dk, pos);
+    const int k = g.r0[2] + (int)(pos - row * nk), o = g.r0[O] + (int)row;
+    const int e0 = g.r0[DIR] + (int)r * run, e1 = min(e0 + run, g.r1[DIR] + 1);
+    long c = DIR == 0 ? cidx(g, e0, o, k) : cidx(g, o, e0, k);
+    double hi[5], h[5], lo[5], qm[5], q0[5], qp[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const double *f = a.P + v * n + c;
+        lo[v] = f[-2 * s];
+        qm[v] = f[-s];
+        q0[v] = f[0];
+        qp[v] = f[s];
+    }
+    muscl_edges<T>(a.lim, lo, qm, q0, h, hi);
+    for (int e = e0;; ++e, c += s) {
+        double qn[5];
+        const bool more = e + 1 < e1;
+#pragma unroll
+        for (int v = 0; v < 5; ++v) qn[v] = more ? a.P[v * n + c + 2 * s] : 0.0;
+        muscl_edges<T>(a.lim, qm, q0, qp, lo, h);
+        T F[5];
+        srhd_face<RIEM, DIR, T>(a, hi, lo, c - s, c, F, a.aux);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            a.F[v * n + c] = F[v];
+            qm[v] = q0[v];
+            q0[v] = qp[v];
+            qp[v] = qn[v];
+            hi[v] = h[v];
+        }
+        if (!more) return;
     }
 }
 

@@ -1,14 +1,50 @@
 // afd_srhd.hip -- SRHD face kernels (MUSCL/PPM/WENO x HLLE/HLLC x x,y x FP64/mixed) and the update with the
 // z faces.
+#include <algorithm>
+
 #include "afd_launch.hpp"
 
 namespace afd {
 
+// MUSCL faces go by runs from RUN_FACES faces on; SLOTS waves of them run at a time (four on each of the
+// 1024 SIMDs), and the length is the one whose rounds of waves take the fewest face times, a run's start
+// counted as START of them (RUN_MAX: longer runs gain nothing and leave the L2s).
+constexpr long RUN_FACES = 3l << 20, RUN_MAX = 32, SLOTS = 4096;
+constexpr double START = 1.5;
+
+static int run_length(long npos, int faces) {
+    int best = 1;
+    double least = 0.0;
+    for (int m = 1; m <= std::min<long>(faces, RUN_MAX); ++m) {
+        const long waves = (npos + 63) / 64 * ((faces + m - 1) / m);
+        const double t = (double)((waves + SLOTS - 1) / SLOTS) * (m + START);
+        if (m == 1 || t < least) {
+            least = t;
+            best = m;
+        }
+    }
+    return best;
+}
+
 template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, hipStream_t s) {
     FaceArgs<T> a = face_args<T>(l);
-    dim3 grid = grid1d(face_count(l.g, l.dir));
-    if (l.dir == 0) hipLaunchKernelGGL((k_face_srhd<RECON, RIEM, 0, T>), grid, dim3(BLOCK), 0, s, a);
-    else hipLaunchKernelGGL((k_face_srhd<RECON, RIEM, 1, T>), grid, dim3(BLOCK), 0, s, a);
+    const Grid &g = l.g;
+    const long count = face_count(g, l.dir);
+    if constexpr (RECON == 0) {
+        if (count >= RUN_FACES) {
+            const int faces = g.r1[l.dir] - g.r0[l.dir] + 1;
+            const long npos = count / faces, nb = (npos + BLOCK - 1) / BLOCK;
+            const int run = run_length(npos, faces);
+            a.dn = make_udiv((unsigned)nb);
+            const dim3 grid((unsigned)(nb * ((faces + run - 1) / run)));
+            if (l.dir == 0) k_face_srhd<RECON, RIEM, 0, T><<<grid, dim3(BLOCK), 0, s>>>(a, run);
+            else k_face_srhd<RECON, RIEM, 1, T><<<grid, dim3(BLOCK), 0, s>>>(a, run);
+            return;
+        }
+    }
+    const dim3 grid = grid1d(count);
+    if (l.dir == 0) k_face_srhd<RECON, RIEM, 0, T><<<grid, dim3(BLOCK), 0, s>>>(a);
+    else k_face_srhd<RECON, RIEM, 1, T><<<grid, dim3(BLOCK), 0, s>>>(a);
 }
 
 template <typename T> static void go_t(const FaceLaunch &l, hipStream_t s) {

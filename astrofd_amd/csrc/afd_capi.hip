@@ -648,7 +648,8 @@ static int pin_draws(afd_ctx *c, const double *draws, size_t n, const double **p
     return AFD_OK;
 }
 
-static int nozzle_fill(afd_ctx *c, const double *draws, int64_t ndraws) {
+// The nozzle's arguments, with the draws in pinned memory
+static int nozzle_args(afd_ctx *c, const double *draws, int64_t ndraws, NozzleArgs *a) {
     if (!c->noz_set) return fail(AFD_ERR_STATE, "nozzle not set (afd_set_nozzle)");
     int64_t need = 0;
     const double *pinned = nullptr;
@@ -658,24 +659,73 @@ static int nozzle_fill(afd_ctx *c, const double *draws, int64_t ndraws) {
             return fail(AFD_ERR_INVALID, "perturbed nozzle needs " + std::to_string(need) + " draws");
         if (int rc = pin_draws(c, draws, (size_t)need, &pinned)) return rc;
     }
-    NozzleArgs a;
+    a->tmpl = c->noz_tmpl;
+    a->idx = c->noz_idx;
+    a->draws = pinned;
+    a->nact = c->noz_nact;
+    a->perturb = need > 0;
+    a->mask = c->noz_mask;
+    a->vamp = c->noz.turb_vamp;
+    a->pamp = c->noz.turb_pamp;
+    return AFD_OK;
+}
+
+static NozzleArgs grid_args(afd_ctx *c) {
+    NozzleArgs a{};
     a.P = c->P[c->cur];
-    a.tmpl = c->noz_tmpl;
-    a.idx = c->noz_idx;
-    a.draws = pinned;
     a.g = c->g;
     a.ng = c->p.ng;
     a.ny_int = c->p.ny;
     a.nz_int = c->p.nz;
-    a.nact = c->noz_nact;
-    a.perturb = need > 0;
-    a.mask = c->noz_mask;
-    a.vamp = c->noz.turb_vamp;
-    a.pamp = c->noz.turb_pamp;
+    return a;
+}
+
+static int nozzle_fill(afd_ctx *c, const double *draws, int64_t ndraws) {
+    NozzleArgs a = grid_args(c);
+    if (int rc = nozzle_args(c, draws, ndraws, &a)) return rc;
     Timed t(c, 4);
     hipLaunchKernelGGL(k_nozzle, grid1d((long)c->p.ng * c->p.ny * c->p.nz), dim3(BLOCK), 0, c->stream, a);
     HIPCHK(hipGetLastError());
-    if (need > 0) HIPCHK(hipEventRecord(c->draws_ev[c->draws_slot], c->stream));
+    if (a.perturb) HIPCHK(hipEventRecord(c->draws_ev[c->draws_slot], c->stream));
+    return AFD_OK;
+}
+
+// Every ghost cell in one launch (k_fill_ghosts), where its sources are interior cells and its element
+// numbers fit 31 bits.
+static bool one_fill(const afd_ctx *c) {
+    const Grid &g = c->g;
+    const long ng = c->p.ng, ring = 2 * ng * (g.nz + c->p.ny), lim = 1l << 31;
+    return ng > 0 && c->p.nx >= 1 && c->p.ny >= ng && c->p.nz >= ng && g.nv * (g.nx - ng) * ring < lim &&
+           g.nv * ng * g.sx < lim;
+}
+
+static int fill_ghosts(afd_ctx *c, const double *draws, int64_t ndraws) {
+    const Grid &g = c->g;
+    FillArgs a{};
+    a.n = grid_args(c);
+    a.nozzle = c->noz_set;
+    if (a.nozzle)
+        if (int rc = nozzle_args(c, draws, ndraws, &a.n)) return rc;
+    const unsigned ng = (unsigned)c->p.ng, ring = 2 * ng * (unsigned)(g.nz + c->p.ny);
+    const unsigned ni = (unsigned)g.nx - ng - (a.nozzle ? ng : 0), plane_int = (unsigned)c->p.ny * c->p.nz;
+    a.bc_y = c->p.bc_y;
+    a.bc_z = c->p.bc_z;
+    a.ring = make_udiv(ring);
+    a.ni = make_udiv(ni);
+    a.plane = make_udiv((unsigned)g.sx);
+    a.ng = make_udiv(ng);
+    a.ng2 = make_udiv(2 * ng);
+    a.plane_int = make_udiv(plane_int);
+    a.nz_int = make_udiv((unsigned)c->p.nz);
+    a.nA = (unsigned)g.nv * ni * ring;
+    a.nB = (unsigned)g.nv * ng * (unsigned)g.sx;
+    a.nC = a.nozzle ? (unsigned)g.nv * ng * plane_int : 0;
+    a.bA = grid1d(a.nA).x;
+    a.bB = grid1d(a.nB).x;
+    Timed t(c, 4);
+    hipLaunchKernelGGL(k_fill_ghosts, dim3(a.bA + a.bB + (a.nC ? grid1d(a.nC).x : 0)), dim3(BLOCK), 0, c->stream, a);
+    HIPCHK(hipGetLastError());
+    if (a.n.perturb) HIPCHK(hipEventRecord(c->draws_ev[c->draws_slot], c->stream));
     return AFD_OK;
 }
 
@@ -705,6 +755,7 @@ extern "C" int afd_apply_nozzle_left_x(afd_ctx *c, const double *draws, int64_t 
 extern "C" int afd_apply_bcs(afd_ctx *c, const double *draws, int64_t ndraws) {
     if (!c) return fail(AFD_ERR_INVALID, "null context");
     HIPCHK(hipSetDevice(c->p.device));
+    if (one_fill(c)) return fill_ghosts(c, draws, ndraws);
     int rc;
     if ((rc = fill_yz(c, 3))) return rc;
     if ((rc = outflow_x(c))) return rc;

@@ -175,27 +175,102 @@ __global__ __launch_bounds__(BLOCK) void k_outflow_x(BcArgs a) {
     b[(long)(g.nx - a.ng + gi) * plane + jk] = b[(long)(g.nx - a.ng - 1) * plane + jk];
 }
 
-__global__ __launch_bounds__(BLOCK) void k_nozzle(NozzleArgs a) {
+// The nozzle's value of variable v in cell c, ghost plane gi and interior (j, k) number jk
+AFD_D void nozzle_value(const NozzleArgs &a, int v, long c, int gi, unsigned jk, unsigned plane) {
 #pragma clang fp contract(off)
+    if (v >= 32 || !((a.mask >> v) & 1u)) return;
+    double val = a.tmpl[(long)v * plane + jk];
+    int rank = a.idx[jk];
+    if (a.perturb && rank >= 0 && v >= 2 && v <= 4) {
+        const double *d = a.draws + 3 * ((long)gi * a.nact + rank);
+        if (v == 2) val = val + a.vamp * (2.0 * d[0] - 1.0);
+        else if (v == 3) val = val + a.vamp * (2.0 * d[1] - 1.0);
+        else val = val * (1.0 + a.pamp * (2.0 * d[2] - 1.0));
+    }
+    a.P[(long)v * a.g.ncell + c] = val;
+}
+
+__global__ __launch_bounds__(BLOCK) void k_nozzle(NozzleArgs a) {
     const Grid &g = a.g;
-    long t = (long)blockIdx.x * BLOCK + threadIdx.x;
-    long plane = (long)a.ny_int * a.nz_int;
-    if (t >= (long)a.ng * plane) return;
-    long jk = t % plane;
-    int gi = (int)(t / plane);
-    int jj = (int)(jk / a.nz_int), kk = (int)(jk % a.nz_int);
-    long c = cidx(g, gi, a.ng + jj, a.ng + kk);
-    for (int v = 0; v < g.nv && v < 32; ++v) {
-        if (!((a.mask >> v) & 1u)) continue;
-        double val = a.tmpl[(long)v * plane + jk];
-        int rank = a.idx[jk];
-        if (a.perturb && rank >= 0 && v >= 2 && v <= 4) {
-            const double *d = a.draws + 3 * ((long)gi * a.nact + rank);
-            if (v == 2) val = val + a.vamp * (2.0 * d[0] - 1.0);
-            else if (v == 3) val = val + a.vamp * (2.0 * d[1] - 1.0);
-            else val = val * (1.0 + a.pamp * (2.0 * d[2] - 1.0));
+    const unsigned t = blockIdx.x * BLOCK + threadIdx.x, plane = (unsigned)a.ny_int * a.nz_int;
+    if (t >= (unsigned)a.ng * plane) return;
+    const unsigned gi = t / plane, jk = t - gi * plane, jj = jk / a.nz_int;
+    const long c = cidx(g, (int)gi, a.ng + (int)jj, a.ng + (int)(jk - jj * a.nz_int));
+    for (int v = 0; v < g.nv && v < 32; ++v) nozzle_value(a, v, c, (int)gi, jk, plane);
+}
+
+// Source index of the y or z fill at position j of an axis of n cells (interior positions: j)
+AFD_D int fill_source(int j, int n, int ng, int bc) {
+    if (j < ng) return bc ? ng : n - 2 * ng + j;
+    if (j >= n - ng) return bc ? n - ng - 1 : ng + (j - (n - ng));
+    return j;
+}
+AFD_D int ghost_pos(int a, int n, int ng) { return a < ng ? a : n - 2 * ng + a; }  // ghost a of 2 ng
+
+// The ghost positions filled from interior position j: [lo0, lo1) and [hi0, hi1)
+struct Images {
+    int lo0, lo1, hi0, hi1;
+};
+AFD_D Images fill_images(int j, int n, int ng, int bc) {
+    const int m = n - 2 * ng;  // interior cells
+    if (bc) return Images{0, j == ng ? ng : 0, n - ng, j == n - ng - 1 ? n : n - ng};
+    return Images{j - m, j - m + (j >= m ? 1 : 0), j + m, j + m + (j < 2 * ng ? 1 : 0)};
+}
+
+__global__ __launch_bounds__(BLOCK) void k_fill_ghosts(FillArgs a) {
+    const Grid &g = a.n.g;
+    const int ng = a.n.ng;
+    double *P = a.n.P;
+    if (blockIdx.x < a.bA) {
+        const unsigned t = blockIdx.x * BLOCK + threadIdx.x;
+        if (t >= a.nA) return;
+        const unsigned q = udiv(a.ring, t), rows = 2u * ng * g.nz;
+        unsigned r = t - q * (rows + 2u * ng * a.n.ny_int);
+        const int first = a.nozzle ? ng : 0, ni = g.nx - ng - first;
+        const unsigned v = udiv(a.ni, q);
+        const int i = first + (int)(q - v * ni);
+        int j, k;
+        if (r < rows) {
+            const unsigned gj = udiv(g.dnz, r);
+            k = (int)(r - gj * g.nz);
+            j = ghost_pos((int)gj, g.ny, ng);
+        } else {
+            r -= rows;
+            const unsigned jj = udiv(a.ng2, r);
+            k = ghost_pos((int)(r - jj * 2u * ng), g.nz, ng);
+            j = ng + (int)jj;
         }
-        a.P[(long)v * g.ncell + c] = val;
+        double *b = P + (long)v * g.ncell;
+        b[cidx(g, i, j, k)] = b[cidx(g, i, fill_source(j, g.ny, ng, a.bc_y), fill_source(k, g.nz, ng, a.bc_z))];
+    } else if (blockIdx.x < a.bA + a.bB) {
+        const unsigned t = (blockIdx.x - a.bA) * BLOCK + threadIdx.x;
+        if (t >= a.nB) return;
+        const unsigned q = udiv(a.plane, t), jk = t - q * (unsigned)g.sx, v = udiv(a.ng, q), ju = udiv(g.dnz, jk);
+        const int i = g.nx - ng + (int)(q - v * ng), j = (int)ju, k = (int)(jk - ju * g.nz);
+        double *b = P + (long)v * g.ncell;
+        b[cidx(g, i, j, k)] =
+            b[cidx(g, g.nx - ng - 1, fill_source(j, g.ny, ng, a.bc_y), fill_source(k, g.nz, ng, a.bc_z))];
+    } else {
+        const unsigned t = (blockIdx.x - a.bA - a.bB) * BLOCK + threadIdx.x;
+        if (t >= a.nC) return;
+        const unsigned plane = (unsigned)a.n.ny_int * a.n.nz_int, q = udiv(a.plane_int, t), jk = t - q * plane;
+        const unsigned v = udiv(a.ng, q), jj = udiv(a.nz_int, jk);
+        const int i = (int)(q - v * ng), j = ng + (int)jj, k = ng + (int)(jk - jj * a.n.nz_int);
+        const long c = cidx(g, i, j, k);
+        if (j < 2 * ng || j >= g.ny - 2 * ng || k < 2 * ng || k >= g.nz - 2 * ng) {
+            double *b = P + (long)v * g.ncell;
+            const double old = b[c];
+            const Images y = fill_images(j, g.ny, ng, a.bc_y), z = fill_images(k, g.nz, ng, a.bc_z);
+            auto row = [&](int jd, bool own) {
+                for (int kd = z.lo0; kd < z.lo1; ++kd) b[cidx(g, i, jd, kd)] = old;
+                for (int kd = z.hi0; kd < z.hi1; ++kd) b[cidx(g, i, jd, kd)] = old;
+                if (!own) b[cidx(g, i, jd, k)] = old;
+            };
+            row(j, true);
+            for (int jd = y.lo0; jd < y.lo1; ++jd) row(jd, false);
+            for (int jd = y.hi0; jd < y.hi1; ++jd) row(jd, false);
+        }
+        nozzle_value(a.n, (int)v, c, i, jk, plane);
     }
 }
 

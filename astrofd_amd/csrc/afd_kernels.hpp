@@ -1768,6 +1768,25 @@ struct NozzleArgs {
 
 __global__ void k_nozzle(NozzleArgs a);
 
+// All ghost cells of a state in one launch: what k_fill_y, k_fill_z, k_outflow_x and (with `nozzle`)
+// k_nozzle leave one after another.  After the y and z fills ghost (i, j, k) holds P(i, J(j), K(k)) with J, K the
+// fills' source indices, which are interior where each axis has at least ng cells (the launcher's rule;
+// with fewer a fill reads ghosts and the four kernels run).  Element ranges, each from a workgroup of its
+// own: the y and z ghosts of the planes up to the last interior one; the +x planes; and the -x planes
+// under the nozzle, one thread per interior (j, k) and variable, which copies the old value to its images
+// before it writes the nozzle's.  The fills are bound by launches up to 64^3, then by partial cache lines;
+// with them (four kernels -> one): 32^3 with a nozzle 13.5 -> 4.0 us, 64^3 RMHD 20 -> 6.8, 128^3 25 -> 13,
+// 160^3 RMHD 34 -> 21, 256^3 periodic 31 -> 23.
+struct FillArgs {
+    NozzleArgs n;                    // also P, the grid and ng
+    int bc_y, bc_z;
+    bool nozzle;
+    UDiv ring, ni, plane, ng, ng2, plane_int, nz_int;  // divisors of the element indices
+    unsigned nA, nB, nC;             // elements of the ranges
+    unsigned bA, bB;                 // workgroups of the first two
+};
+__global__ void k_fill_ghosts(FillArgs a);
+
 // The driver's post-step sources (solvers/srhd3d_mpi_muscl.py:324-326), pointwise over the
 // interior, applied in that order to each cell in one pass: cooling/heating
 // (core/source_terms.py:5-28), two-temperature relaxation (:30-55), H/He ion chemistry

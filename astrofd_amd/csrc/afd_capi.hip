@@ -896,6 +896,7 @@ static UpdLaunch upd_launch(afd_ctx *c, const double *Pin, const double *P0, dou
     a.gr = c->p.gr_metric == 0 ? 0 : (c->p.gr_metric == 1 ? 1 : 2);
     a.gr_x0 = c->p.gr_x0;
     a.amax = nullptr;
+    a.amax_clear = nullptr;
     a.sbox = c->sbox;
     a.gr_mass = c->p.gr_mass;
     a.gr_gfac = c->p.gr_metric == 0 ? 0.0 : c->p.gr_gamma / (c->p.gr_gamma - 1.0);
@@ -919,9 +920,9 @@ extern "C" int afd_step(afd_ctx *c, double dt) {
         int rc = run_faces(c, c->P[src], c->nb == 5 ? 2 : (c->fused ? 1 : -1));
         if (rc) return rc;
         UpdLaunch l = upd_launch(c, c->P[src], c->P[in], c->P[dst], s, nst, dt);
-        if (c->nb == 5 && s == nst - 1) {  // SRHD: the next step's CFL speed from the last stage
-            HIPCHK(hipMemsetAsync(c->amax_dev, 0, AMAX_BOX_BYTES, c->stream));
-            l.a.amax = c->amax_dev;
+        if (c->nb == 5) {  // the next step's CFL speed from the last stage
+            if (s == 0) l.a.amax_clear = c->amax_dev;
+            if (s == nst - 1) l.a.amax = c->amax_dev;
         }
         if (c->repair_qcount)
             HIPCHK(hipMemsetAsync(c->repair_qcount, 0, sizeof(unsigned) * QUEUE_SLOTS, c->stream));

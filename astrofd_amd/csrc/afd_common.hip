@@ -453,31 +453,36 @@ __global__ __launch_bounds__(BLOCK) void k_max_speed_shell(const double *P, Grid
                                                             double gfac, unsigned long long *amax) {
     // range [1, n-1) per axis, box [lo, hi) inside it: slabs i outside (all j, k), then i inside
     // with j outside (all k), then i, j inside with k outside
-    const long bi = g.nx - 2, bj = g.ny - 2, bk = g.nz - 2;
-    const long ni = b.hi[0] - b.lo[0], nj = b.hi[1] - b.lo[1], nk = b.hi[2] - b.lo[2];
-    const long oi = bi - ni, oj = bj - nj, ok = bk - nk;
-    const long nA = oi * bj * bk, nB = ni * oj * bk, nC = ni * nj * ok;
-    long t = (long)blockIdx.x * BLOCK + threadIdx.x;
+    const unsigned bi = g.nx - 2, bj = g.ny - 2, bk = g.nz - 2;
+    const unsigned ni = b.hi[0] - b.lo[0], nj = b.hi[1] - b.lo[1], nk = b.hi[2] - b.lo[2];
+    const unsigned oi = bi - ni, oj = bj - nj, ok = bk - nk;
+    const unsigned nA = oi * bj * bk, nB = ni * oj * bk, nC = ni * nj * ok;
+    unsigned t = blockIdx.x * BLOCK + threadIdx.x;
     double v = 0.0;
     if (t < nA + nB + nC) {
-        auto out = [&](long p, int ax) { return p < b.lo[ax] - 1 ? 1 + p : b.hi[ax] + (p - (b.lo[ax] - 1)); };
-        long i, j, k;
+        auto out_pos = [&](unsigned p, int ax) {
+            return (int)p < b.lo[ax] - 1 ? 1 + (int)p : b.hi[ax] + ((int)p - (b.lo[ax] - 1));
+        };
+        int i, j, k;
         if (t < nA) {
-            k = 1 + t % bk;
-            j = 1 + (t / bk) % bj;
-            i = out(t / (bk * bj), 0);
+            const unsigned r = t / bk, q = r / bj;
+            k = 1 + (int)(t - r * bk);
+            j = 1 + (int)(r - q * bj);
+            i = out_pos(q, 0);
         } else if (t < nA + nB) {
             t -= nA;
-            k = 1 + t % bk;
-            j = out((t / bk) % oj, 1);
-            i = b.lo[0] + t / (bk * oj);
+            const unsigned r = t / bk, q = r / oj;
+            k = 1 + (int)(t - r * bk);
+            j = out_pos(r - q * oj, 1);
+            i = b.lo[0] + (int)q;
         } else {
             t -= nA + nB;
-            k = out(t % ok, 2);
-            j = b.lo[1] + (t / ok) % nj;
-            i = b.lo[0] + t / (ok * nj);
+            const unsigned r = t / ok, q = r / nj;
+            k = out_pos(t - r * ok, 2);
+            j = b.lo[1] + (int)(r - q * nj);
+            i = b.lo[0] + (int)q;
         }
-        const long c = cidx(g, (int)i, (int)j, (int)k);
+        const long c = cidx(g, i, j, k);
         v = srhd_cell_speed(gamma, gfac, P[c], P[g.ncell + c], P[2 * g.ncell + c], P[3 * g.ncell + c],
                             P[4 * g.ncell + c]);
     }

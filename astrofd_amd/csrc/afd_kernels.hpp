@@ -1014,6 +1014,7 @@ template <typename F> struct UpdArgs {
     unsigned long long *amax;     // SRHD last stage: max characteristic speed over sbox of the new
                                   //   primitives, as the bits of a double >= 0 (atomicMax into
                                   //   AMAX_SLOTS slots), or null
+    unsigned long long *amax_clear;  // SRHD first stage: those slots, to be zeroed, or null
     SpeedBox sbox;
 };
 
@@ -1440,6 +1441,10 @@ constexpr int ZCELLS = 62;  // cells a wave updates
 template <typename F>
 AFD_D void update_faces_z(const FaceArgs<F> &fa, const UpdArgs<F> &ua, int recon, int riem, bool rhs_only) {
     const Grid &g = ua.g;
+    if (ua.amax_clear) {
+        for (unsigned t = blockIdx.x * BLOCK + threadIdx.x; t < AMAX_SLOTS; t += gridDim.x * BLOCK)
+            ua.amax_clear[t * AMAX_STRIDE] = 0ull;
+    }
     const int lane = threadIdx.x & 63;
     const long n = g.ncell, c = (long)(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * ZCELLS + lane - 1;
     const bool live = lane >= 1 && lane <= ZCELLS && c < n;
@@ -1775,7 +1780,7 @@ __global__ void k_nozzle(NozzleArgs a);
 // own: the y and z ghosts of the planes up to the last interior one; the +x planes; and the -x planes
 // under the nozzle, one thread per interior (j, k) and variable, which copies the old value to its images
 // before it writes the nozzle's.  The fills are bound by launches up to 64^3, then by partial cache lines;
-// with them (four kernels -> one): 32^3 with a nozzle 13.5 -> 4.0 us, 64^3 RMHD 20 -> 6.8, 128^3 25 -> 13,
+// the four kernels and this one: 32^3 with a nozzle 13.5 -> 4.0 us, 64^3 RMHD 20 -> 6.8, 128^3 25 -> 13,
 // 160^3 RMHD 34 -> 21, 256^3 periodic 31 -> 23.
 struct FillArgs {
     NozzleArgs n;                    // also P, the grid and ng
@@ -1861,7 +1866,9 @@ __global__ void k_diss_store(DissArgs a, double *P);
 // the last stage of a step (cell_update) or by k_max_speed_box into the first AMAX_SLOTS slots,
 // and the rest, taken by k_max_speed_shell after the fills into the next AMAX_SLOTS slots.  Both
 // atomicMax the bits of a double >= 0.  k_amax_finish (one block of BLOCK threads) writes
-// max(all slots, floor) as a double to out and zeroes the shell's slots for the next call.
+// max(all slots, floor) as a double to out and zeroes the shell's slots for the next call; the box's
+// slots are zeroed by a step's first stage (update_faces_z).  The end in the shell's last workgroup
+// instead: its fences cost more than the launch (32^3 7.3 us for 4.1 + 2.6, 256^3 95 for 15 + 4).
 __global__ void k_max_speed_box(const double *P, Grid g, SpeedBox b, double gamma, double gfac,
                                 unsigned long long *amax);
 __global__ void k_max_speed_shell(const double *P, Grid g, SpeedBox b, double gamma, double gfac,

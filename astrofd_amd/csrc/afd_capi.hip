@@ -810,20 +810,29 @@ static int run_faces(afd_ctx *c, const double *P, int skip) {
     // launched here) goes first
     const int order_carried[3] = {2, 0, 1}, order_plain[3] = {0, 1, 2}, order_div[3] = {1, 2, 0};
     const int *order = c->dmode && skip != 1 ? order_div : (c->carried ? order_carried : order_plain);
+    // small grids: x and y in one launch (and z, where the x faces do not need what it stores)
+    const bool merge = !c->shared_edges && face_count(c->g, 0) < MERGE_FACES, merge_z = merge && c->nb == 9 && !c->carried;
+    FaceLaunch d3[3] = {l, l, l};
     bool first = true;
     for (int n = 0; n < 3; ++n) {
-        int d = order[n];
+        const int d = order[n];
         if (d == skip) continue;
-        l.dfirst = first;
+        FaceLaunch &f = d3[d];
+        f.dfirst = first;
         first = false;
-        l.dir = d;
-        l.idn = (float)(1.0 / (d == 0 ? c->p.dx : (d == 1 ? c->p.dy : c->p.dz)));
-        l.F = Fd[d];
-        l.Fcar = (c->carried && d == 0) ? c->Fxc : nullptr;
-        l.zs = c->carried ? c->zs : nullptr;
-        l.aux = c->passive_flux ? c->aux[d] : nullptr;
+        f.dir = d;
+        f.idn = (float)(1.0 / (d == 0 ? c->p.dx : (d == 1 ? c->p.dy : c->p.dz)));
+        f.F = Fd[d];
+        f.Fcar = (c->carried && d == 0) ? c->Fxc : nullptr;
+        f.zs = c->carried ? c->zs : nullptr;
+        f.aux = c->passive_flux ? c->aux[d] : nullptr;
+    }
+    for (int n = 0; n < 3; ++n) {
+        const int d = order[n];
+        if (d == skip || (merge && d == 1) || (merge_z && d == 2)) continue;
+        const FaceLaunch *y = merge && d == 0 ? &d3[1] : nullptr, *z = merge_z && d == 0 ? &d3[2] : nullptr;
         Timed t(c, d);
-        hipError_t e = (c->nb == 9) ? launch_face_rmhd(l, c->stream) : launch_face_srhd(l, c->stream);
+        hipError_t e = c->nb == 9 ? launch_face_rmhd(d3[d], y, z, c->stream) : launch_face_srhd(d3[d], y, c->stream);
         if (e != hipSuccess) return fail(AFD_ERR_HIP, std::string("face kernel: ") + hipGetErrorString(e));
     }
     return AFD_OK;

@@ -535,11 +535,12 @@ __global__ __launch_bounds__(BLOCK) void k_reduce_sum_u64(const unsigned long lo
     if (threadIdx.x == 0) out[0] = red[0];
 }
 
-template <typename T> void launch_face_rmhd_t(const FaceLaunch &l, hipStream_t s);
+template <typename T>
+void launch_face_rmhd_t(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z, hipStream_t s);
 
-hipError_t launch_face_rmhd(const FaceLaunch &l, hipStream_t s) {
-    if (l.mixed) launch_face_rmhd_t<float>(l, s);
-    else launch_face_rmhd_t<double>(l, s);
+hipError_t launch_face_rmhd(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z, hipStream_t s) {
+    if (l.mixed) launch_face_rmhd_t<float>(l, y, z, s);
+    else launch_face_rmhd_t<double>(l, y, z, s);
     return hipGetLastError();
 }
 

@@ -52,8 +52,9 @@ inline long face_count(const Grid &g, int dir) {
     return n;
 }
 
-hipError_t launch_face_srhd(const FaceLaunch &l, hipStream_t s);
-hipError_t launch_face_rmhd(const FaceLaunch &l, hipStream_t s);
+// The faces of one direction; y, z not null: l's (x) faces with those in one launch (k_faces_srhd, k_faces_rmhd).
+hipError_t launch_face_srhd(const FaceLaunch &l, const FaceLaunch *y, hipStream_t s);
+hipError_t launch_face_rmhd(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z, hipStream_t s);
 
 // RMHD stage update / rhs-only launch.  flux pointers typed by `mixed`.
 struct UpdLaunch {

@@ -63,7 +63,16 @@ template <int RIEM> static void go_weno_xy_march(const FaceLaunch &l, hipStream_
     else hipLaunchKernelGGL((k_face_rmhd_weno_march<RIEM, 1, true>), grid, block, 0, s, a);
 }
 
-template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, hipStream_t s) {
+template <int RECON, int RIEM, typename T>
+static void go(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z, hipStream_t s) {
+    if (y) {  // l: the x faces
+        const unsigned nx = grid1d(face_count(l.g, 0)).x, ny = grid1d(face_count(l.g, 1)).x;
+        const unsigned nz = z ? grid1d(face_count(l.g, 2)).x : 0;
+        const FaceArgs<T> x = face_args<T>(l);
+        hipLaunchKernelGGL((k_faces_rmhd<RECON, RIEM, T>), dim3(nx + ny + nz), dim3(BLOCK), 0, s, x, face_args<T>(*y),
+                           z ? face_args<T>(*z) : x, nx, ny);
+        return;
+    }
     if constexpr (RECON == 2 && sizeof(T) == 4) {
         if (l.D) {  // the context decided: shared edges, below 2^29 cells
             if (l.dir == 2) go_weno_z_div<RIEM>(l, s);
@@ -83,21 +92,23 @@ template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, h
     else hipLaunchKernelGGL((k_face_rmhd<RECON, RIEM, 2, T>), grid, dim3(BLOCK), 0, s, a);
 }
 
-template <typename T> void launch_face_rmhd_t(const FaceLaunch &l, hipStream_t s) {
+template <typename T>
+void launch_face_rmhd_t(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z, hipStream_t s) {
     int key = l.recon * 3 + (l.riemann < 0 ? 0 : (l.riemann > 2 ? 2 : l.riemann));
     switch (key) {
-        case 0: go<0, 0, T>(l, s); break;
-        case 1: go<0, 1, T>(l, s); break;
-        case 2: go<0, 2, T>(l, s); break;
-        case 3: go<1, 0, T>(l, s); break;
-        case 4: go<1, 1, T>(l, s); break;
-        case 5: go<1, 2, T>(l, s); break;
-        case 6: go<2, 0, T>(l, s); break;
-        case 7: go<2, 1, T>(l, s); break;
-        default: go<2, 2, T>(l, s); break;
+        case 0: go<0, 0, T>(l, y, z, s); break;
+        case 1: go<0, 1, T>(l, y, z, s); break;
+        case 2: go<0, 2, T>(l, y, z, s); break;
+        case 3: go<1, 0, T>(l, y, z, s); break;
+        case 4: go<1, 1, T>(l, y, z, s); break;
+        case 5: go<1, 2, T>(l, y, z, s); break;
+        case 6: go<2, 0, T>(l, y, z, s); break;
+        case 7: go<2, 1, T>(l, y, z, s); break;
+        default: go<2, 2, T>(l, y, z, s); break;
     }
 }
 
-template void launch_face_rmhd_t<AFD_RMHD_T>(const FaceLaunch &l, hipStream_t s);
+template void launch_face_rmhd_t<AFD_RMHD_T>(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z,
+                                             hipStream_t s);
 
 }  // namespace afd

@@ -6,10 +6,10 @@
 
 namespace afd {
 
-// MUSCL faces go by runs from RUN_FACES faces on; SLOTS waves of them run at a time (four on each of the
+// MUSCL faces go by runs from MERGE_FACES faces on; SLOTS waves of them run at a time (four on each of the
 // 1024 SIMDs), and the length is the one whose rounds of waves take the fewest face times, a run's start
 // counted as START of them (RUN_MAX: longer runs gain nothing and leave the L2s).
-constexpr long RUN_FACES = 3l << 20, RUN_MAX = 32, SLOTS = 4096;
+constexpr long RUN_MAX = 32, SLOTS = 4096;
 constexpr double START = 1.5;
 
 static int run_length(long npos, int faces) {
@@ -26,12 +26,17 @@ static int run_length(long npos, int faces) {
     return best;
 }
 
-template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, hipStream_t s) {
+template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, const FaceLaunch *y, hipStream_t s) {
     FaceArgs<T> a = face_args<T>(l);
     const Grid &g = l.g;
     const long count = face_count(g, l.dir);
+    if (y) {  // l: the x faces
+        const unsigned nx = grid1d(count).x, ny = grid1d(face_count(g, 1)).x;
+        hipLaunchKernelGGL((k_faces_srhd<RECON, RIEM, T>), dim3(nx + ny), dim3(BLOCK), 0, s, a, face_args<T>(*y), nx);
+        return;
+    }
     if constexpr (RECON == 0) {
-        if (count >= RUN_FACES) {
+        if (count >= MERGE_FACES) {
             const int faces = g.r1[l.dir] - g.r0[l.dir] + 1;
             const long npos = count / faces, nb = (npos + BLOCK - 1) / BLOCK;
             const int run = run_length(npos, faces);
@@ -47,21 +52,21 @@ template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, h
     else k_face_srhd<RECON, RIEM, 1, T><<<grid, dim3(BLOCK), 0, s>>>(a);
 }
 
-template <typename T> static void go_t(const FaceLaunch &l, hipStream_t s) {
+template <typename T> static void go_t(const FaceLaunch &l, const FaceLaunch *y, hipStream_t s) {
     int key = l.recon * 2 + (l.riemann == 1 ? 1 : 0);
     switch (key) {
-        case 0: go<0, 0, T>(l, s); break;
-        case 1: go<0, 1, T>(l, s); break;
-        case 2: go<1, 0, T>(l, s); break;
-        case 3: go<1, 1, T>(l, s); break;
-        case 4: go<2, 0, T>(l, s); break;
-        default: go<2, 1, T>(l, s); break;
+        case 0: go<0, 0, T>(l, y, s); break;
+        case 1: go<0, 1, T>(l, y, s); break;
+        case 2: go<1, 0, T>(l, y, s); break;
+        case 3: go<1, 1, T>(l, y, s); break;
+        case 4: go<2, 0, T>(l, y, s); break;
+        default: go<2, 1, T>(l, y, s); break;
     }
 }
 
-hipError_t launch_face_srhd(const FaceLaunch &l, hipStream_t s) {
-    if (l.mixed) go_t<float>(l, s);
-    else go_t<double>(l, s);
+hipError_t launch_face_srhd(const FaceLaunch &l, const FaceLaunch *y, hipStream_t s) {
+    if (l.mixed) go_t<float>(l, y, s);
+    else go_t<double>(l, y, s);
     return hipGetLastError();
 }
 

@@ -117,7 +117,9 @@ typedef struct afd_stats {
     uint64_t invalid;         /* RMHD cells whose recovery was invalid (hydro guess kept) */
     uint64_t learned_ok;      /* RMHD cells solved from the learned guess (acceptance test passed) */
     uint64_t c2p_cells;       /* cells converted */
-    double ms_face[3];        /* summed HIP-event time of the x, y, z face kernels (timing on) */
+    double ms_face[3];        /* summed HIP-event time of the x, y, z face kernels (timing on);
+                                 launches of several directions count as x, and the SRHD z faces are
+                                 part of the update */
     double ms_update;         /* summed time of the stage-update (+ con2prim) kernel */
     double ms_other;          /* BCs, passives, reductions */
     uint64_t launches_face[3], launches_update;

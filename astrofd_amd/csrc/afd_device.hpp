@@ -40,12 +40,12 @@ template <typename T> AFD_D T pymax(T a, T b) { return (b > a) ? b : a; }
 // reciprocal is shared, a quotient takes four (product, exact residual, correction and the special
 // cases) and nothing is scaled: the same operations on the same values, so the same bits.  The scaling
 // acts only near the ends of the exponent range: divisors are to lie in [2^-960, 2^1020] (or be 0, inf
-// or NaN), quotients below 2^-970 may differ in their last bit and one beyond the largest double is NaN,
-// not inf.  Every FP64 division and square root of the physics goes through Div, fsqrt and finvsqrt: the
-// FP64 kernels are bound by vector instructions, of which the scaling was a tenth (RMHD WENO5 faces of a
-// 160^3 grid: 385, 358 and 344 us with it, 333, 303 and 286 without; SRHD MUSCL faces at 256^3: 498 and
-// 472 us).  FP32: the hardware reciprocal (about 1 ulp), whose error is far below the FP32 rounding the
-// mixed path already accepts.
+// or NaN), numerators and quotients below 2^-900 may cost the last bit and a quotient beyond the largest
+// double is NaN, not inf.  Every FP64 division and square root of the physics goes through Div, fsqrt
+// and finvsqrt: the FP64 kernels are bound by vector instructions, of which the scaling was a tenth
+// (RMHD WENO5 faces of a 160^3 grid: 385, 358 and 344 us with it, 333, 303 and 286 without; SRHD MUSCL
+// faces at 256^3: 498 and 472 us).  FP32: the hardware reciprocal (about 1 ulp), whose error is far below
+// the FP32 rounding the mixed path already accepts.
 template <typename T> struct Div;
 template <> struct Div<double> {
     double b, y;
@@ -194,6 +194,10 @@ template <typename T> AFD_D void ppm_reconstruct(T qm2, T qm1, T q0, T qp1, T qp
 // indicators have every fused multiply-add written out: left to the compiler, which product is fused
 // follows what the neighbouring edges share, so a change elsewhere in a kernel would move its results by
 // an ulp.  fuse3: the product of 3 q0 - 4 qp1 that is fused (both are exact to an ulp).
+// The weights' numerators carry a power of two, which leaves every bit of the weights as it is: without it
+// the sum of 1 / IS^2 falls below the smallest divisor that Div takes (2^-960) where a variable jumps by
+// more than 2^240, and the edge is NaN; with it the weights hold as far as IS^2 does.
+constexpr double WENO_UP = 0x1p500;
 template <typename T>
 AFD_D void weno5_indicators(T qm2, T qm1, T q0, T qp1, T qp2, bool fuse3, T &IS0, T &IS1, T &IS2) {
 #pragma clang fp contract(off)
@@ -208,9 +212,9 @@ template <typename T> AFD_D T weno5_left(T qm2, T qm1, T q0, T qp1, T qp2, bool 
     const T eps = T(1e-12);
     T IS0, IS1, IS2;
     weno5_indicators(qm2, qm1, q0, qp1, qp2, fuse3, IS0, IS1, IS2);
-    T a0 = fdiv(T(0.1), sq(eps + IS0));
-    T a1 = fdiv(T(0.6), sq(eps + IS1));
-    T a2 = fdiv(T(0.3), sq(eps + IS2));
+    T a0 = fdiv(T(0.1 * WENO_UP), sq(eps + IS0));
+    T a1 = fdiv(T(0.6 * WENO_UP), sq(eps + IS1));
+    T a2 = fdiv(T(0.3 * WENO_UP), sq(eps + IS2));
     T s = a0 + a1 + a2;
     const Div<T> by(s);
     T w0 = by(a0), w1 = by(a1), w2 = by(a2);
@@ -229,7 +233,8 @@ AFD_D double weno5_edge(double qm2, double qm1, double q0, double qp1, double qp
     const double p0 = fma(11.0 / 6.0, q0, fma(c13, qm2, -((7.0 / 6.0) * qm1)));
     const double p1 = fma(c13, qp1, fma(c56, q0, -(c16 * qm1)));
     const double p2 = fma(-c16, qp2, right ? fma(c56, qp1, c13 * q0) : fma(c13, q0, c56 * qp1));
-    const double a0 = fdiv(0.1, sq(1e-12 + IS0)), a1 = fdiv(0.6, sq(1e-12 + IS1)), a2 = fdiv(0.3, sq(1e-12 + IS2));
+    const double a0 = fdiv(0.1 * WENO_UP, sq(1e-12 + IS0)), a1 = fdiv(0.6 * WENO_UP, sq(1e-12 + IS1)),
+                 a2 = fdiv(0.3 * WENO_UP, sq(1e-12 + IS2));
     const Div<double> by(a0 + a1 + a2);
     return fma(by(a2), p2, fma(by(a0), p0, by(a1) * p1));
 }

@@ -961,7 +961,8 @@ AFD_D double passive_weno_edge(double qm2, double qm1, double q0, double qp1, do
     const double IS0 = fma(c, sq((qm2 - 2.0 * qm1) + q0), 0.25 * sq(fma(3.0, q0, qm2 - 4.0 * qm1)));
     const double IS1 = fma(0.25, sq(qm1 - qp1), c * sq((qm1 - 2.0 * q0) + qp1));
     const double IS2 = fma(c, sq((q0 - 2.0 * qp1) + qp2), 0.25 * sq(fma(-4.0, qp1, 3.0 * q0) + qp2));
-    const double a0 = fdiv(0.1, sq(eps + IS0)), a1 = fdiv(0.6, sq(eps + IS1)), a2 = fdiv(0.3, sq(eps + IS2));
+    const double a0 = fdiv(0.1 * WENO_UP, sq(eps + IS0)), a1 = fdiv(0.6 * WENO_UP, sq(eps + IS1)),
+                 a2 = fdiv(0.3 * WENO_UP, sq(eps + IS2));
     const Div<double> by(a0 + a1 + a2);
     return fma(by(a2), p2, fma(by(a0), p0, by(a1) * p1));
 }

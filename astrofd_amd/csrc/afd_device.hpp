@@ -850,18 +850,22 @@ AFD_D double rmhd_f_of_Z(const RmhdC2PParams &c, double Z, double D, double tau,
     return tau_calc - tau;
 }
 
-// Newton on Z from Z_start (core/rmhd_core.py:273-290): returns true when |f| < tol
+// Newton on Z (core/rmhd_core.py:273-290), its steps it .. maxit - 1: returns true when |f| < tol.  it is
+// left at the steps done, at `never` where the slope vanished (no later step is taken then).
 template <bool FAST = false>
-AFD_D bool rmhd_newton(const RmhdC2PParams &c, double &Z, double D, double tau, double B2, double SB, double S2,
-                       double tol, int maxit, C2PStats &st) {
-    for (int it = 0; it < maxit; ++it) {
+AFD_D bool rmhd_newton_steps(const RmhdC2PParams &c, double &Z, double D, double tau, double B2, double SB, double S2,
+                             double tol, int &it, int maxit, int never, C2PStats &st) {
+    for (; it < maxit; ++it) {
         double f = rmhd_f_of_Z<FAST>(c, Z, D, tau, B2, SB, S2);
         st.newton_iters += 1;
         if (fabs(f) < tol) return true;
         double eps = 1e-6 * pymax(1.0, Z);
         double fp = rmhd_f_of_Z<FAST>(c, Z + eps, D, tau, B2, SB, S2);
         double dfdZ = fdiv(fp - f, eps);
-        if (dfdZ == 0.0) return false;
+        if (dfdZ == 0.0) {
+            it = never;
+            return false;
+        }
         double dZ = fdiv(-f, dfdZ);
         if (dZ > 0.5 * Z) dZ = 0.5 * Z;
         if (dZ < -0.5 * Z) dZ = -0.5 * Z;
@@ -869,6 +873,12 @@ AFD_D bool rmhd_newton(const RmhdC2PParams &c, double &Z, double D, double tau, 
         if (Z < SMALL) Z = SMALL;
     }
     return false;
+}
+template <bool FAST = false>
+AFD_D bool rmhd_newton(const RmhdC2PParams &c, double &Z, double D, double tau, double B2, double SB, double S2,
+                       double tol, int maxit, C2PStats &st) {
+    int it = 0;
+    return rmhd_newton_steps<FAST>(c, Z, D, tau, B2, SB, S2, tol, it, maxit, maxit, st);
 }
 
 // Recover the primitives from Z (core/rmhd_core.py:320-341); the hydro guess q0 replaces invalid
@@ -925,63 +935,78 @@ AFD_D bool rmhd_recover(const RmhdC2PParams &c, double Z, const double *U, doubl
     return true;
 }
 
-// core/rmhd_core.py:248-341 (hydro guess, FD-Newton from Z0 then Z1, bisection, recovery)
-// count: the hydro guess's iteration count is wanted (hydro_c2p).
+// What the root f(Z) = 0 of a state is sought with
+struct RmhdRoot {
+    double D, tau, B2, SB, S2;
+    AFD_D double Z1() const { return pymax(D + tau + B2, SMALL); }
+    AFD_D double tol() const { return 1e-10 * pymax(1.0, tau); }
+};
+constexpr int RMHD_NEWTON_STEPS = 50;
+
+// core/rmhd_core.py:248-341: hydro guess q0, FD-Newton from Z0 then Z1, bisection, recovery.  First the
+// guess and Z0.  count: the hydro guess's iteration count is wanted (hydro_c2p).
 template <bool FAST = false>
-AFD_D void rmhd_c2p(const RmhdC2PParams &c, const double *U, double *q, C2PStats &st, bool count) {
+AFD_D double rmhd_c2p_start(const RmhdC2PParams &c, const double *U, double *q0, RmhdRoot &r, C2PStats &st, bool count) {
     double D = U[0], Sx = U[1], Sy = U[2], Sz = U[3], tau = U[4], Bx = U[5], By = U[6], Bz = U[7];
-    double B2 = Bx * Bx + By * By + Bz * Bz;
-    double SB = Sx * Bx + Sy * By + Sz * Bz;
-    double S2 = Sx * Sx + Sy * Sy + Sz * Sz;
-    double tau_h = tau - 0.5 * B2;
+    r.D = D;
+    r.tau = tau;
+    r.B2 = Bx * Bx + By * By + Bz * Bz;
+    r.SB = Sx * Bx + Sy * By + Sz * Bz;
+    r.S2 = Sx * Sx + Sy * Sy + Sz * Sz;
+    double tau_h = tau - 0.5 * r.B2;
     if (tau_h < SMALL) tau_h = SMALL;
-    double Uh[5] = {D, Sx, Sy, Sz, tau_h}, q0[5];
+    double Uh[5] = {D, Sx, Sy, Sz, tau_h};
     hydro_c2p<FAST>(c.gamma, c.gfac, c.p_max, c.v_max, Uh, q0, st, count);
     double vmax2 = c.v_max * c.v_max;
     double v20 = q0[1] * q0[1] + q0[2] * q0[2] + q0[3] * q0[3];
     if (v20 >= vmax2) v20 = vmax2 - 1e-14;
     double W0 = finvsqrt(1.0 - v20);
     double h0 = 1.0 + fdiv(c.gfac * q0[4], pymax(q0[0], SMALL));
-    double Z0 = pymax(q0[0] * h0 * W0 * W0, SMALL);
-    double Z1 = pymax(D + tau + B2, SMALL);
-    double tol = 1e-10 * pymax(1.0, tau);
-    double Z = Z0;
-    bool ok = rmhd_newton<FAST>(c, Z, D, tau, B2, SB, S2, tol, 50, st);
-    if (!ok) {
-        Z = Z1;
-        ok = rmhd_newton<FAST>(c, Z, D, tau, B2, SB, S2, tol, 50, st);
+    return pymax(q0[0] * h0 * W0 * W0, SMALL);
+}
+// ... Newton from Z1 and the bisection, where Newton from Z0 has failed: Z
+template <bool FAST = false> AFD_D double rmhd_c2p_second(const RmhdC2PParams &c, const RmhdRoot &r, C2PStats &st) {
+    const double D = r.D, tau = r.tau, B2 = r.B2, SB = r.SB, S2 = r.S2, Z1 = r.Z1(), tol = r.tol();
+    double Z = Z1;
+    if (rmhd_newton<FAST>(c, Z, D, tau, B2, SB, S2, tol, RMHD_NEWTON_STEPS, st)) return Z;
+    st.flags |= 2;
+    double Zmin = SMALL;
+    double Zmax = pymax(pymax(Z, Z1), 1.0);
+    double fmin = rmhd_f_of_Z<FAST>(c, Zmin, D, tau, B2, SB, S2);
+    double fmax = rmhd_f_of_Z<FAST>(c, Zmax, D, tau, B2, SB, S2);
+    for (int it = 0; it < 40; ++it) {
+        if (fmin * fmax <= 0.0) break;
+        Zmax *= 2.0;
+        fmax = rmhd_f_of_Z<FAST>(c, Zmax, D, tau, B2, SB, S2);
     }
-    if (!ok) {
-        st.flags |= 2;
-        double Zmin = SMALL;
-        double Zmax = pymax(pymax(Z, Z1), 1.0);
-        double fmin = rmhd_f_of_Z<FAST>(c, Zmin, D, tau, B2, SB, S2);
-        double fmax = rmhd_f_of_Z<FAST>(c, Zmax, D, tau, B2, SB, S2);
-        for (int it = 0; it < 40; ++it) {
-            if (fmin * fmax <= 0.0) break;
-            Zmax *= 2.0;
-            fmax = rmhd_f_of_Z<FAST>(c, Zmax, D, tau, B2, SB, S2);
-        }
-        if (fmin * fmax <= 0.0) {
-            for (int it = 0; it < 60; ++it) {
-                double Zmid = 0.5 * (Zmin + Zmax);
-                double fmid = rmhd_f_of_Z<FAST>(c, Zmid, D, tau, B2, SB, S2);
-                if (fabs(fmid) < tol) {
-                    Z = Zmid;
-                    break;
-                }
-                if (fmin * fmid <= 0.0) {
-                    Zmax = Zmid;
-                    fmax = fmid;
-                } else {
-                    Zmin = Zmid;
-                    fmin = fmid;
-                }
-                Z = 0.5 * (Zmin + Zmax);
+    if (fmin * fmax <= 0.0) {
+        for (int it = 0; it < 60; ++it) {
+            double Zmid = 0.5 * (Zmin + Zmax);
+            double fmid = rmhd_f_of_Z<FAST>(c, Zmid, D, tau, B2, SB, S2);
+            if (fabs(fmid) < tol) {
+                Z = Zmid;
+                break;
             }
+            if (fmin * fmid <= 0.0) {
+                Zmax = Zmid;
+                fmax = fmid;
+            } else {
+                Zmin = Zmid;
+                fmin = fmid;
+            }
+            Z = 0.5 * (Zmin + Zmax);
         }
     }
-    rmhd_recover<FAST>(c, Z, U, B2, SB, q0, q, st);
+    return Z;
+}
+template <bool FAST = false>
+AFD_D void rmhd_c2p(const RmhdC2PParams &c, const double *U, double *q, C2PStats &st, bool count) {
+    double q0[5];
+    RmhdRoot r;
+    double Z = rmhd_c2p_start<FAST>(c, U, q0, r, st, count);
+    if (!rmhd_newton<FAST>(c, Z, r.D, r.tau, r.B2, r.SB, r.S2, r.tol(), RMHD_NEWTON_STEPS, st))
+        Z = rmhd_c2p_second<FAST>(c, r, st);
+    rmhd_recover<FAST>(c, Z, U, r.B2, r.SB, q0, q, st);
 }
 
 // Learned-guess con2prim: FD-Newton (the reference's iteration) from the network's Z0, accepted by a

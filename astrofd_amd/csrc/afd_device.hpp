@@ -750,6 +750,14 @@ struct C2PStats {
 // grows (W falls with p when E >= 0, so rho stays above SMALL) and the loop ends in the fallback, whose
 // result does not depend on where p stood.  Stage update of a moving SRHD flow at 256^3: 1.24 -> 0.87
 // ms in FP64 (181 x 127 x 143 mixed: 0.26 -> 0.14 ms); results bitwise those of the full loop.
+//
+// Below the root p falls instead, by the half that a step may take, for some 40 steps to 1e-12: where p_max
+// cuts its start (a jet's inflow), a few cells of a grid whose waves all others wait for.  With Wx the
+// Lorentz factor at p = 0 (or of v_max), the largest there is below p, and D, E >= 0,
+//   f(p') >= E - D Wx + p' - Gamma/(Gamma-1) p' Wx^2   for every p' <= p,
+// and where that exceeds p' / 2 at p it does so at each smaller p'.  Then the halvings run without f.  The
+// room for rounding grows with Wx^2, as the error of 1 / (1 - v^2) does.  Stage update of a 32^3 SRHD jet
+// 21.8 -> 13.5 us, 128 x 96 x 96 58.5 -> 58.1, RMHD 64^3 32.3 -> 31.8.
 template <bool FAST = false>
 AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const double *U, double *q, C2PStats &st,
                      bool count) {
@@ -787,7 +795,28 @@ AFD_D void hydro_c2p(double g, double gfac, double p_max, double v_max, const do
             ++it;
             break;
         }
+        const bool halved = dp == -0.5 * p;
         p = p_new;
+        if (halved && E >= 0.0 && D >= 0.0) {
+            double vx2 = ddiv<FAST>(S2, E * E + SMALL);
+            if (!(vx2 < vmax2)) vx2 = vmax2;
+            const double Wx = dinvsqrt<FAST>(1.0 - vx2), DW = D * Wx, gW2 = gfac * Wx * Wx;
+            if (E - DW - (gW2 - 0.5) * p > 1e-12 * Wx * Wx * (E + p + DW + gW2 * p)) {
+                for (++it; it < 60; ++it) {
+                    dp = -0.5 * p;
+                    p_new = p + dp;
+                    if (p_new < SMALL) p_new = SMALL;
+                    ok = fabs(dp) < 1e-12 * pymax(1.0, p_new);
+                    if (ok || p_new == p) {
+                        p = p_new;
+                        ++it;
+                        break;
+                    }
+                    p = p_new;
+                }
+                break;
+            }
+        }
         if (!count && dp > 0.0 && E >= 0.0 && rho >= 2.0 * SMALL && p > 1e-11 &&
             (gfac - 1.0) * p - (E - D) > 1e-11 * (1.0 + p + E + D))
             break;

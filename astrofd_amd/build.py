@@ -46,6 +46,17 @@ UNITS = [
 ]
 
 
+# The FP64 quotients and roots by themselves, for the tests
+ARITH_CHECK = os.path.join(ROOT, "tests", "hip", "libarith_check.so")
+
+
+def build_arith_check():
+    """Compile tests/hip/arith_check.hip; nothing where the tests are not shipped."""
+    src = os.path.join(ROOT, "tests", "hip", "arith_check.hip")
+    if os.path.exists(src):
+        subprocess.run([HIPCC] + HIPFLAGS + ["-shared", src, "-o", ARITH_CHECK], check=True, capture_output=True)
+
+
 def _compile(unit, verbose):
     src, extra = unit[0], unit[1]
     name = unit[2] if len(unit) > 2 else os.path.splitext(src)[0]

@@ -74,7 +74,8 @@ template <typename T> AFD_D T fdiv(T a, T b) { return Div<T>(b)(a); }
 // Functions", ch. 9), a correction by the exact residual, and div_fixup for 0, inf and NaN; 9
 // instructions for 18.  The iteration leaves g and h (half of 1 / sqrt(x)) with errors below 2^-46 (the
 // hardware's start has 2^-24), the correction g with 2^-92, so that the rounding can go wrong for one
-// x in 2^38 (none in 8.6e9 random ones).  FP32: the hardware's (about 1 ulp).
+// x in 2^38 (none in 8.6e9 random ones).  Below zero div_fixup makes -inf of the iteration's NaN (it takes a
+// NaN quotient of finite operands for an overflow): nan_below_zero.  FP32: the hardware's (about 1 ulp).
 AFD_D double sqrt_core(double x, double &h) {
 #pragma clang fp contract(off)
     const double y = __builtin_amdgcn_rsq(x);
@@ -85,10 +86,14 @@ AFD_D double sqrt_core(double x, double &h) {
     h = fma(h, r, h);
     return fma(fma(-g, g, x), h, g);
 }
+// r, or NaN where x < 0 (two instructions: with the upper half of a NaN every lower half is one)
+AFD_D double nan_below_zero(double x, double r) {
+    return __hiloint2double(x < 0.0 ? 0x7ff80000 : __double2hiint(r), __double2loint(r));
+}
 template <typename T> AFD_D T fsqrt(T x) {
     double h;
     const double g = sqrt_core(x, h);
-    return __builtin_amdgcn_div_fixup(g, 1.0, x);
+    return nan_below_zero(x, __builtin_amdgcn_div_fixup(g, 1.0, x));
 }
 template <> AFD_D float fsqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
 // 1 / sqrt(x) rounded as 1.0 / sqrt(x) is (both operations), same x: the reciprocal is the root's h
@@ -99,7 +104,7 @@ AFD_D double finvsqrt(double x) {
     double h;
     const double g = sqrt_core(x, h);
     const double y = h * (2.0 + 0x1p-51);
-    return __builtin_amdgcn_div_fixup(fma(fma(-g, y, 1.0), y, y), x, 1.0);
+    return nan_below_zero(x, __builtin_amdgcn_div_fixup(fma(fma(-g, y, 1.0), y, y), x, 1.0));
 }
 // FP64 division / inverse square root.  FAST = false: IEEE (the plain path rounds as the
 // reference).  FAST = true (mixed path: con2prim, Lorentz factors): the hardware reciprocal / reciprocal square

@@ -40,12 +40,13 @@ template <typename T> AFD_D T pymax(T a, T b) { return (b > a) ? b : a; }
 // reciprocal is shared, a quotient takes four (product, exact residual, correction and the special
 // cases) and nothing is scaled: the same operations on the same values, so the same bits.  The scaling
 // acts only near the ends of the exponent range: divisors are to lie in [2^-960, 2^1020] (or be 0, inf
-// or NaN), numerators and quotients below 2^-900 may cost the last bit and a quotient beyond the largest
-// double is NaN, not inf.  Every FP64 division and square root of the physics goes through Div, fsqrt
-// and finvsqrt: the FP64 kernels are bound by vector instructions, of which the scaling was a tenth
-// (RMHD WENO5 faces of a 160^3 grid: 385, 358 and 344 us with it, 333, 303 and 286 without; SRHD MUSCL
-// faces at 256^3: 498 and 472 us).  FP32: the hardware reciprocal (about 1 ulp), whose error is far below
-// the FP32 rounding the mixed path already accepts.
+// or NaN), and numerators and quotients below 2^-900 may cost the last bit.  A quotient beyond the largest
+// double is inf, as con2prim's caps on v^2 need it: the correction is NaN there, of which div_fixup makes an
+// infinity of the quotient's sign; one within two ulp of the largest double may be inf too.  Every FP64
+// division and square root of the physics goes through Div, fsqrt and finvsqrt: the FP64 kernels are bound
+// by vector instructions, of which the scaling was a tenth (RMHD WENO5 faces of a 160^3 grid: 385, 358 and
+// 344 us with it, 333, 303 and 286 without; SRHD MUSCL faces at 256^3: 498 and 472 us).  FP32: the hardware
+// reciprocal (about 1 ulp), whose error is far below the FP32 rounding the mixed path already accepts.
 template <typename T> struct Div;
 template <> struct Div<double> {
     double b, y;

@@ -1,5 +1,5 @@
-"""The FP64 roots of afd_device.hpp (fsqrt, finvsqrt), element by element, bit for bit against the IEEE ones of
-numpy (tests/hip/arith_check.hip evaluates them)."""
+"""The FP64 quotients and roots of afd_device.hpp (fdiv, fsqrt, finvsqrt), element by element, bit for bit against
+the IEEE ones of numpy (tests/hip/arith_check.hip evaluates them)."""
 import ctypes
 import os
 
@@ -12,7 +12,8 @@ from .gpu_helpers import make_domain
 
 pytestmark = pytest.mark.gpu
 
-SQRT, RSQRT = 1, 2  # arith_check's operations
+QUOTIENT, SQRT, RSQRT = 0, 1, 2  # arith_check's operations
+MAX = np.finfo(np.float64).max
 
 
 def evaluate(op, a, b=None):
@@ -60,3 +61,56 @@ def test_p2c_outside_the_light_cone():
     with make_domain("rmhd", (9, 12, 12, 12), 2, gamma=4.0 / 3.0, v_max=2.0) as d:
         U = d.p2c(q)
     assert np.array_equal(np.isnan(U), np.isnan(ref)) and np.array_equal(np.isinf(U), np.isinf(ref))
+
+
+def test_quotients():
+    """Over the ranges that Div states; quotients within two ulp of the largest double aside, which may be inf."""
+    r = np.random.default_rng(1)
+    n = 1 << 20
+    b = numbers(r, n, -960, 1020)
+    a = np.where(r.random(n) < 0.5, numbers(r, n, -900, 1024),
+                 np.ldexp(numbers(r, n, 0, 1), np.clip(np.frexp(b)[1] + r.integers(-60, 60, n), -900, 1023)))
+    a[::1001] = 0.0
+    with np.errstate(all="ignore"):
+        ref = a / b
+        ok = (np.abs(ref) >= 2.0 ** -900) | (a == 0.0)
+    ok &= ~((np.abs(ref) > MAX * (1.0 - 2.0 ** -51)) & np.isfinite(ref))
+    assert ok.sum() > n // 2
+    assert same(evaluate(QUOTIENT, a, b)[ok], ref[ok])
+
+
+def test_quotients_beyond_the_largest_double():
+    """Infinite, as a / b: con2prim's caps on v^2 rely on it."""
+    r = np.random.default_rng(2)
+    n = 1 << 18
+    b = numbers(r, n, -900, 1000)
+    a = np.ldexp(numbers(r, n, 0, 1), np.clip(np.frexp(b)[1] + r.integers(1013, 1030, n), -900, 1023))
+    with np.errstate(over="ignore"):
+        ref = a / b
+    ok = np.isinf(ref) | (np.abs(ref) <= MAX * (1.0 - 2.0 ** -51))
+    assert np.isinf(ref).sum() > n // 8 and ok.sum() > 0.99 * n and np.isfinite(a).all()
+    assert same(evaluate(QUOTIENT, a, b)[ok], ref[ok])
+
+
+def test_quotients_of_specials():
+    v = np.array([0.0, 1.0, 3.0, 1e-12, 1e300, 2.0 ** -900, np.inf, np.nan])
+    v = np.concatenate([v, -v])
+    a, b = (x.ravel() for x in np.meshgrid(v, v))
+    with np.errstate(all="ignore"):
+        ref = a / b
+    assert same(evaluate(QUOTIENT, a, b), ref)
+
+
+@pytest.mark.parametrize("op", [SQRT, RSQRT])
+def test_roots(op):
+    """Random arguments, squares, and arguments whose root lies next to a power of two.  (One argument in 2^38
+    may round wrongly: 1 in 10^5 for a draw of this size.)"""
+    r = np.random.default_rng(5)
+    n = 1 << 20
+    k = r.integers(-12, 13, 1 << 14)
+    y = np.where(k < 0, 1.0 + k * 2.0 ** -53, 1.0 + k * 2.0 ** -52)  # neighbours of 1
+    x = np.concatenate([np.abs(numbers(r, n, -760, 1024)), (1.0 + r.random(n)) ** 2, np.arange(1.0, 65537.0),
+                        np.ldexp(y, 2 * r.integers(-380, 511, y.size)), np.ldexp(y * y, 2 * r.integers(-380, 511, y.size))])
+    x = x[x >= 2.0 ** -760]
+    ref = np.sqrt(x) if op == SQRT else 1.0 / np.sqrt(x)
+    assert same(evaluate(op, x), ref)

@@ -30,7 +30,7 @@ _D = ctypes.POINTER(ctypes.c_double)
 
 
 class AfdError(RuntimeError):
-    pass
+    code = AFD_OK  # the call's AFD_ERR_*
 
 
 class Params(ctypes.Structure):
@@ -173,7 +173,9 @@ def exported_symbols():
 def check(rc, what=""):
     if rc != 0:
         msg = load().afd_last_error().decode(errors="replace")
-        raise AfdError(f"{what}: error {rc}: {msg}")
+        e = AfdError(f"{what}: error {rc}: {msg}")
+        e.code = rc
+        raise e
 
 
 def dptr(a):

@@ -15,10 +15,10 @@ def _physics(pr):
 
 
 def _fill(pr, ng, call):
-    d = _ctx.domain(_physics(pr), pr.shape, ng=ng)
-    d.set_prim(pr)
-    call(d)
-    pr[...] = d.get_prim()
+    with _ctx.domain(_physics(pr), pr.shape, ng=ng) as d:
+        d.set_prim(pr)
+        call(d)
+        pr[...] = d.get_prim()
 
 
 def apply_periodic_yz(pr, ng):

@@ -11,8 +11,8 @@ def apply_ion_chemistry(pr, dt, cfg):
         return pr
     if pr.shape[0] <= int(cfg.get("CHEM_OFFSET", 0)) + 2:
         return pr
-    d = _ctx.source_domain(pr.shape, int(cfg.get("NG", 2)))
-    d.set_prim(pr)
-    d.ion_chemistry(dt, chem_from_settings(cfg))
-    pr[...] = d.get_prim()
+    with _ctx.source_domain(pr.shape, int(cfg.get("NG", 2))) as d:
+        d.set_prim(pr)
+        d.ion_chemistry(dt, chem_from_settings(cfg))
+        pr[...] = d.get_prim()
     return pr

@@ -11,8 +11,8 @@ def apply_causal_dissipation(pr, dt, dx, dy, dz, cfg):
         return pr
     if pr.shape[0] < 15:
         return pr
-    d = _ctx.source_domain(pr.shape, int(cfg.get("NG", 2)), dxyz=(dx, dy, dz))
-    d.set_prim(pr)
-    d.causal_dissipation(dt, diss_from_settings(cfg))
-    pr[...] = d.get_prim()
+    with _ctx.source_domain(pr.shape, int(cfg.get("NG", 2)), dxyz=(dx, dy, dz)) as d:
+        d.set_prim(pr)
+        d.causal_dissipation(dt, diss_from_settings(cfg))
+        pr[...] = d.get_prim()
     return pr

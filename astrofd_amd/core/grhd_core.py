@@ -30,16 +30,16 @@ def compute_rhs_grhd(pr, dx, dy, dz, offs_x, ng):
     """core/grhd_core.py:20-75: the flat RHS of the configured reconstruction with the flux velocities
     divided by the Kerr-Schild lapse (ORTHONORMAL_FLUX, Schwarzschild or Kerr-Schild), plus the
     lapse-gradient sources for every metric but Minkowski."""
-    d = _ctx.domain("hydro", pr.shape, (dx, dy, dz), ng=ng, gr=_gr(offs_x))
-    d.set_prim(pr)
-    return d.compute_rhs()
+    with _ctx.domain("hydro", pr.shape, (dx, dy, dz), ng=ng, gr=_gr(offs_x)) as d:
+        d.set_prim(pr)
+        return d.compute_rhs()
 
 
 def _step(pr, dx, dy, dz, dt, offs_x, ng, order):
-    d = _ctx.domain("hydro", pr.shape, (dx, dy, dz), rk_order=order, ng=ng, gr=_gr(offs_x))
-    d.set_prim(pr)
-    d.step(dt)
-    return d.get_prim()
+    with _ctx.domain("hydro", pr.shape, (dx, dy, dz), rk_order=order, ng=ng, gr=_gr(offs_x)) as d:
+        d.set_prim(pr)
+        d.step(dt)
+        return d.get_prim()
 
 
 def step_ssprk2(pr, dx, dy, dz, dt, offs_x, ng):

@@ -28,12 +28,12 @@ def apply_nozzle_left_x(pr, dx, dy, dz, ny_loc, nz_loc, y0, z0, rng, cfg):
     """core/nozzle.py:27-92, in place on pr.  `rng` (numpy Generator) supplies the perturbation
     draws in the reference's order when NOZZLE_PERTURB is not "none"."""
     phys = _physics(pr)
-    d = _ctx.domain(phys, pr.shape, (dx, dy, dz), ng=int(cfg["NG"]))
     if ny_loc != pr.shape[2] - 2 * int(cfg["NG"]) or nz_loc != pr.shape[3] - 2 * int(cfg["NG"]):
         raise ValueError("ny_loc / nz_loc must be the interior y / z sizes of pr")
     n = nozzle_from_settings(dict(cfg, JET_CENTER=[0.0, float(y0), float(z0)]))
-    L.check(d.lib.afd_set_nozzle(d.h, ctypes.byref(n)), "afd_set_nozzle")
-    d.nozzle_set = True
-    d.set_prim(pr)
-    d.apply_nozzle_left_x(rng)
-    pr[...] = d.get_prim()
+    with _ctx.domain(phys, pr.shape, (dx, dy, dz), ng=int(cfg["NG"])) as d:
+        L.check(d.lib.afd_set_nozzle(d.h, ctypes.byref(n)), "afd_set_nozzle")
+        d.nozzle_set = True
+        d.set_prim(pr)
+        d.apply_nozzle_left_x(rng)
+        pr[...] = d.get_prim()

@@ -15,22 +15,24 @@ def configure(params):
 def prim_to_cons_rmhd(rho, vx, vy, vz, p, Bx, By, Bz, psi, gamma=None):
     """core/rmhd_core.py:138-168 -> (D, Sx, Sy, Sz, tau, Bx, By, Bz, psi)."""
     q, shape = _ctx.as_batch((rho, vx, vy, vz, p, Bx, By, Bz, psi), 9)
-    return _ctx.unbatch(_ctx.pointwise("rmhd", gamma).p2c(q), shape)
+    with _ctx.pointwise("rmhd", gamma) as d:
+        return _ctx.unbatch(d.p2c(q), shape)
 
 
 def cons_to_prim_rmhd(D, Sx, Sy, Sz, tau, Bx, By, Bz, psi):
     """core/rmhd_core.py:249-341 -> (rho, vx, vy, vz, p, Bx, By, Bz, psi)."""
     u, shape = _ctx.as_batch((D, Sx, Sy, Sz, tau, Bx, By, Bz, psi), 9)
-    return _ctx.unbatch(_ctx.pointwise("rmhd").c2p(u), shape)
+    with _ctx.pointwise("rmhd") as d:
+        return _ctx.unbatch(d.c2p(u), shape)
 
 
 def _rhs(pr, recon, dx, dy, dz):
     s = _ctx.settings("rmhd")
     if str(s.get("RECON", "muscl")).lower() != recon:
         _ctx.configure("rmhd", dict(s, RECON=recon))
-    d = _ctx.domain("rmhd", pr.shape, (dx, dy, dz))
-    d.set_prim(pr)
-    return d.compute_rhs()
+    with _ctx.domain("rmhd", pr.shape, (dx, dy, dz)) as d:
+        d.set_prim(pr)
+        return d.compute_rhs()
 
 
 def compute_rhs_rmhd(pr, nx, ny, nz, dx, dy, dz):
@@ -49,10 +51,10 @@ def compute_rhs_weno(pr, nx, ny, nz, dx, dy, dz):
 
 
 def _step(pr, dx, dy, dz, dt, order):
-    d = _ctx.domain("rmhd", pr.shape, (dx, dy, dz), rk_order=order)
-    d.set_prim(pr)
-    d.step(dt)
-    return d.get_prim()
+    with _ctx.domain("rmhd", pr.shape, (dx, dy, dz), rk_order=order) as d:
+        d.set_prim(pr)
+        d.step(dt)
+        return d.get_prim()
 
 
 def step_ssprk2(pr, dx, dy, dz, dt):

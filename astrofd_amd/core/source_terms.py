@@ -13,10 +13,10 @@ def apply_cooling_heating(pr, dt, cfg):
     cool, heat = float(cfg.get("COOLING_LAMBDA", 0.0)), float(cfg.get("HEATING_RATE", 0.0))
     if cool == 0.0 and heat == 0.0:
         return pr
-    d = _ctx.source_domain(pr.shape, int(cfg.get("NG", 2)))
-    d.set_prim(pr)
-    d.cooling_heating(dt, cool, heat, float(cfg.get("P_MAX", 1.0)))
-    pr[...] = d.get_prim()
+    with _ctx.source_domain(pr.shape, int(cfg.get("NG", 2))) as d:
+        d.set_prim(pr)
+        d.cooling_heating(dt, cool, heat, float(cfg.get("P_MAX", 1.0)))
+        pr[...] = d.get_prim()
     return pr
 
 
@@ -29,8 +29,8 @@ def apply_two_temperature(pr, dt, cfg):
     tau = float(cfg.get("TEI_TAU", 0.5))
     if pr.shape[0] < off + 2 or tau <= 0.0:
         return pr
-    d = _ctx.source_domain(pr.shape, int(cfg.get("NG", 2)), two_temp=(off, tau))
-    d.set_prim(pr)
-    d.two_temperature(dt)
-    pr[...] = d.get_prim()
+    with _ctx.source_domain(pr.shape, int(cfg.get("NG", 2)), two_temp=(off, tau)) as d:
+        d.set_prim(pr)
+        d.two_temperature(dt)
+        pr[...] = d.get_prim()
     return pr

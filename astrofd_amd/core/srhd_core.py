@@ -20,22 +20,24 @@ def configure(params):
 def prim_to_cons(rho, vx, vy, vz, p, gamma=GAMMA):
     """core/srhd_core.py:47-59 -> (D, Sx, Sy, Sz, tau)."""
     q, shape = _ctx.as_batch((rho, vx, vy, vz, p), 5)
-    return _ctx.unbatch(_ctx.pointwise("hydro", gamma).p2c(q), shape)
+    with _ctx.pointwise("hydro", gamma) as d:
+        return _ctx.unbatch(d.p2c(q), shape)
 
 
 def cons_to_prim(D, Sx, Sy, Sz, tau, gamma=GAMMA):
     """core/srhd_core.py:62-131 -> (rho, vx, vy, vz, p)."""
     u, shape = _ctx.as_batch((D, Sx, Sy, Sz, tau), 5)
-    return _ctx.unbatch(_ctx.pointwise("hydro", gamma).c2p(u), shape)
+    with _ctx.pointwise("hydro", gamma) as d:
+        return _ctx.unbatch(d.c2p(u), shape)
 
 
 def _rhs(pr, recon, dx, dy, dz):
     s = _ctx.settings("hydro")
     if str(s.get("RECON", "muscl")).lower() != recon:
         _ctx.configure("hydro", dict(s, RECON=recon))
-    d = _ctx.domain("hydro", pr.shape, (dx, dy, dz))
-    d.set_prim(pr)
-    return d.compute_rhs()
+    with _ctx.domain("hydro", pr.shape, (dx, dy, dz)) as d:
+        d.set_prim(pr)
+        return d.compute_rhs()
 
 
 def compute_rhs_muscl(pr, nx, ny, nz, dx, dy, dz):
@@ -55,16 +57,16 @@ def compute_rhs_weno(pr, nx, ny, nz, dx, dy, dz):
 
 def max_char_speed(pr, nx, ny, nz):
     """core/srhd_core.py:1268-1281: max |lambda| over [1, n-1)^3."""
-    d = _ctx.domain("hydro", pr.shape)
-    d.set_prim(pr)
-    return d.max_char_speed()
+    with _ctx.domain("hydro", pr.shape) as d:
+        d.set_prim(pr)
+        return d.max_char_speed()
 
 
 def _step(pr, dx, dy, dz, dt, order):
-    d = _ctx.domain("hydro", pr.shape, (dx, dy, dz), rk_order=order)
-    d.set_prim(pr)
-    d.step(dt)
-    return d.get_prim()
+    with _ctx.domain("hydro", pr.shape, (dx, dy, dz), rk_order=order) as d:
+        d.set_prim(pr)
+        d.step(dt)
+        return d.get_prim()
 
 
 def step_ssprk2(pr, dx, dy, dz, dt):

@@ -92,13 +92,14 @@ struct afd_ctx {
     size_t scratch_cap = 0;
     // pinned host memory: a block (from its first use on) of small arrays on their way up and down
     // (PIN_BYTES each) and the CFL speed and counts (written by the kernels), and the nozzle draws of the
-    // last DRAW_SLOTS fills (read by the kernel)
+    // last DRAW_SLOTS fills (read by the kernel; draws_dev without pinned memory)
     char *pin = nullptr;
     bool pin_up_used = false;
     double *host_out = nullptr;
     double *draws_pin[DRAW_SLOTS] = {};
     hipEvent_t draws_ev[DRAW_SLOTS] = {};
-    size_t draws_cap = 0;
+    size_t draws_cap = 0, draws_dev_cap = 0;
+    double *draws_dev = nullptr;
     int draws_slot = 0;
     bool retained = false;
     std::vector<void *> allocs;
@@ -160,6 +161,19 @@ __global__ __launch_bounds__(BLOCK) static void k_copy_words(const unsigned *src
 static bool pin_ready(afd_ctx *c) {
     if (!c->pin && (c->pin = xfer_pin_get())) c->host_out = (double *)(c->pin + 2 * PIN_BYTES);
     return c->pin != nullptr;
+}
+
+// Where a kernel leaves one 8-byte result: pinned memory, which the host reads once the stream is idle, or,
+// where there is none to be had, a device word that result_get copies.
+static double *result_word(afd_ctx *c) { return pin_ready(c) ? c->host_out : c->diag_out; }
+static hipError_t result_get(afd_ctx *c, const double *word, void *out) {
+    if (word == c->diag_out) {
+        hipError_t e = hipMemcpyAsync(out, word, 8, hipMemcpyDeviceToHost, c->stream);
+        return e == hipSuccess ? hipStreamSynchronize(c->stream) : e;
+    }
+    hipError_t e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) memcpy(out, word, 8);
+    return e;
 }
 
 static void copy_words(afd_ctx *c, const void *src, void *dst, size_t bytes) {
@@ -626,7 +640,8 @@ static int outflow_x(afd_ctx *c) {
 // The caller's draws into one of DRAW_SLOTS pinned buffers, which the nozzle kernel reads over the
 // host link (each value once), without waiting for the stream: the host draws the next fill's numbers
 // while the device steps (the wait at each fill left it idle meanwhile).  A buffer is reused once the
-// event after its kernel has passed.
+// event after its kernel has passed.  Where there is no pinned memory to be had they go to a device buffer,
+// and the fill waits.
 static int pin_draws(afd_ctx *c, const double *draws, size_t n, const double **pinned) {
     if (n > c->draws_cap) {
         for (int d = 0; d < DRAW_SLOTS; ++d) {
@@ -636,8 +651,20 @@ static int pin_draws(afd_ctx *c, const double *draws, size_t n, const double **p
         }
         c->draws_cap = 0;
         for (int d = 0; d < DRAW_SLOTS; ++d) {
-            HIPCHK(hipHostMalloc((void **)&c->draws_pin[d], n * 8, 0));
             if (!c->draws_ev[d]) HIPCHK(hipEventCreateWithFlags(&c->draws_ev[d], hipEventDisableTiming));
+            if (hipHostMalloc((void **)&c->draws_pin[d], n * 8, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                c->draws_pin[d] = nullptr;
+                if (n > c->draws_dev_cap) {
+                    c->draws_dev_cap = 0;
+                    ALLOC(c, c->draws_dev, n * 8);
+                    c->draws_dev_cap = n;
+                }
+                HIPCHK(hipMemcpyAsync(c->draws_dev, draws, n * 8, hipMemcpyHostToDevice, c->stream));
+                HIPCHK(hipStreamSynchronize(c->stream));
+                *pinned = c->draws_dev;
+                return AFD_OK;
+            }
         }
         c->draws_cap = n;
     }
@@ -648,7 +675,7 @@ static int pin_draws(afd_ctx *c, const double *draws, size_t n, const double **p
     return AFD_OK;
 }
 
-// The nozzle's arguments, with the draws in pinned memory
+// The nozzle's arguments, with the draws where its kernel can read them
 static int nozzle_args(afd_ctx *c, const double *draws, int64_t ndraws, NozzleArgs *a) {
     if (!c->noz_set) return fail(AFD_ERR_STATE, "nozzle not set (afd_set_nozzle)");
     int64_t need = 0;
@@ -1119,7 +1146,7 @@ extern "C" int afd_post_step_sources(afd_ctx *c, double dt, const afd_sources *s
 extern "C" int afd_max_char_speed(afd_ctx *c, double *amax) {
     if (!c || !amax) return fail(AFD_ERR_INVALID, "afd_max_char_speed: null argument");
     HIPCHK(hipSetDevice(c->p.device));
-    if (!pin_ready(c)) return fail(AFD_ERR_NOMEM, "no pinned memory for the result");
+    double *word = result_word(c);
     const double gfac = c->p.gamma / (c->p.gamma - 1.0);
     const Grid &g = c->g;
     const SpeedBox &b = c->sbox;
@@ -1140,27 +1167,24 @@ extern "C" int afd_max_char_speed(afd_ctx *c, double *amax) {
             hipLaunchKernelGGL(k_max_speed_shell, grid1d(range - inner), dim3(BLOCK), 0, c->stream,
                                (const double *)c->P[c->cur], g, b, c->p.gamma, gfac,
                                c->amax_dev + AMAX_SLOTS * AMAX_STRIDE);
-        hipLaunchKernelGGL(k_amax_finish, dim3(1), dim3(BLOCK), 0, c->stream, c->amax_dev, SMALL,
-                           c->host_out);  // pinned: no copy after the kernel
+        hipLaunchKernelGGL(k_amax_finish, dim3(1), dim3(BLOCK), 0, c->stream, c->amax_dev, SMALL, word);
         HIPCHK(hipGetLastError());
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    *amax = c->host_out[0];
+    HIPCHK(result_get(c, word, amax));
     return AFD_OK;
 }
 
 extern "C" int afd_count_nonfinite(afd_ctx *c, int64_t *count) {
     if (!c || !count) return fail(AFD_ERR_INVALID, "afd_count_nonfinite: null argument");
     HIPCHK(hipSetDevice(c->p.device));
-    if (!pin_ready(c)) return fail(AFD_ERR_NOMEM, "no pinned memory for the result");
+    double *word = result_word(c);
     long n = c->g.ncell * c->p.nv;
     hipLaunchKernelGGL(k_count_nonfinite, dim3(c->red_blocks), dim3(BLOCK), 0, c->stream,
                        (const double *)c->P[c->cur], n, c->cnt_partial);
     hipLaunchKernelGGL(k_reduce_sum_u64, dim3(1), dim3(BLOCK), 0, c->stream,
-                       (const unsigned long long *)c->cnt_partial, c->red_blocks, (unsigned long long *)c->host_out);
+                       (const unsigned long long *)c->cnt_partial, c->red_blocks, (unsigned long long *)word);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->stream));
-    *count = *(const int64_t *)c->host_out;
+    HIPCHK(result_get(c, word, count));
     return AFD_OK;
 }
 

@@ -95,6 +95,7 @@ struct afd_ctx {
     // last DRAW_SLOTS fills (read by the kernel; draws_dev without pinned memory)
     char *pin = nullptr;
     bool pin_up_used = false;
+    long small_transfers = 0;
     double *host_out = nullptr;
     double *draws_pin[DRAW_SLOTS] = {};
     hipEvent_t draws_ev[DRAW_SLOTS] = {};
@@ -158,8 +159,13 @@ __global__ __launch_bounds__(BLOCK) static void k_copy_words(const unsigned *src
     for (unsigned i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) dst[i] = src[i];
 }
 
+// A context takes a closed one's block at once, and has a new one locked at its fifth small transfer: locking and
+// unlocking the pages take 30 us, a transfer through them saves 5.  A state converted on a context opened and closed
+// around it: 192 us with the block locked at the first transfer, 160 without; there and back 225 and 207; three
+// times there and back 325, and 349 with the block from the fifth of the twelve transfers on.
 static bool pin_ready(afd_ctx *c) {
-    if (!c->pin && (c->pin = xfer_pin_get())) c->host_out = (double *)(c->pin + 2 * PIN_BYTES);
+    if (!c->pin && (c->pin = xfer_pin_get(++c->small_transfers > 4)))
+        c->host_out = (double *)(c->pin + 2 * PIN_BYTES);
     return c->pin != nullptr;
 }
 
@@ -210,8 +216,8 @@ static hipError_t copy_down(afd_ctx *c, void *host, const void *dev, size_t byte
 static hipError_t copy_down2(afd_ctx *c, void *host, const void *dev, size_t bytes, void *host2, const void *dev2,
                              size_t bytes2) {
     if (bytes2 > PIN_BYTES || !pin_ready(c)) {
-        hipError_t e = copy_down(c, host, dev, bytes);
-        return e == hipSuccess ? copy_down(c, host2, dev2, bytes2) : e;
+        hipError_t e = xfer_d2h(host, dev, bytes, c->stream, false);
+        return e == hipSuccess ? xfer_d2h(host2, dev2, bytes2, c->stream) : e;
     }
     char *pin = c->pin + PIN_BYTES;
     const bool both = bytes + bytes2 <= PIN_BYTES;

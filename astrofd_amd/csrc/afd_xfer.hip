@@ -223,7 +223,7 @@ void xfer_retain() {
     ++g_refs;
 }
 
-char *xfer_pin_get() {
+char *xfer_pin_get(bool lock) {
     {
         std::lock_guard<std::mutex> l(g_mu);
         for (char *&b : g_pins)
@@ -233,6 +233,7 @@ char *xfer_pin_get() {
                 return r;
             }
     }
+    if (!lock) return nullptr;
     void *p = nullptr;
     if (hipHostMalloc(&p, PIN_BLOCK, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
@@ -270,8 +271,8 @@ void xfer_release() {
     if (p && p->pid == getpid()) delete p;  // a forked child has no threads to join
 }
 
-hipError_t xfer_d2h(void *host, const void *dev, size_t bytes, hipStream_t s) {
-    return copy(true, host, (void *)dev, bytes, s, true);
+hipError_t xfer_d2h(void *host, const void *dev, size_t bytes, hipStream_t s, bool wait) {
+    return copy(true, host, (void *)dev, bytes, s, wait);
 }
 hipError_t xfer_h2d(void *dev, const void *host, size_t bytes, hipStream_t s, bool wait) {
     return copy(false, (void *)host, dev, bytes, s, wait);

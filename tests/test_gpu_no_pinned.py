@@ -40,16 +40,38 @@ def results():
     return out
 
 
-def test_without_pinned_memory(tmp_path):
+def refusing(tmp_path, call):
+    """What `call` (of this file) returns in a process of its own that gets no page-locked memory, and how often it
+    asked for some."""
     src, lib = os.path.join(ROOT, "tests", "hip", "no_pinned.c"), str(tmp_path / "no_pinned.so")
     subprocess.run(["cc", "-shared", "-fPIC", "-O1", src, "-o", lib], check=True)
     # the stand-in is found before the runtime's function: it is loaded before the library that calls it
     code = ("import ctypes, sys; s = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)\n"
             "import numpy as np; from tests import test_gpu_no_pinned as t\n"
-            "np.savez(%r, **t.results(), refused=s.no_pinned_refused())\n") % (lib, str(tmp_path / "out.npz"))
+            "out = t.%s()\n"
+            "np.savez(%r, **out, refused=s.no_pinned_refused())\n") % (lib, call, str(tmp_path / "out.npz"))
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, timeout=90, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
-    got, ref = np.load(tmp_path / "out.npz"), results()
+    return np.load(tmp_path / "out.npz")
+
+
+def conversions():
+    """Two small batches, there and back, on a context each."""
+    from tests.gpu_helpers import make_domain
+    q = np.tile([1.0, 0.1, 0.2, 0.0, 0.1], (50, 1))
+    for _ in range(2):
+        with make_domain("hydro", (5, 12, 12, 12), 2) as d:
+            d.c2p(d.p2c(q), with_iters=True)
+    return {}
+
+
+def test_a_context_for_one_conversion_locks_no_pages(tmp_path):
+    """Locking them takes longer than the batch gains by it."""
+    assert refusing(tmp_path, "conversions")["refused"] == 0
+
+
+def test_without_pinned_memory(tmp_path):
+    got, ref = refusing(tmp_path, "results"), results()
     assert got["refused"] >= 4
     assert ref["hydro_nan"] > 0
     for k, v in ref.items():

@@ -317,9 +317,10 @@ class Domain:
     def c2p(self, cons, with_iters=False):
         cons = L.f64c(cons).reshape(-1, self.nb)
         out = np.empty_like(cons)
-        it = np.zeros(cons.shape[0], dtype=np.int32)
+        it = np.zeros(cons.shape[0], dtype=np.int32) if with_iters else None
         L.check(self.lib.afd_c2p_batch(self.h, cons.shape[0], L.dptr(cons), L.dptr(out),
-                                       it.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))), "afd_c2p_batch")
+                                       it.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)) if with_iters else None),
+                "afd_c2p_batch")
         return (out, it) if with_iters else out
 
     # ---- diagnostics (utils/diagnostics.py)

@@ -844,7 +844,8 @@ static int run_faces(afd_ctx *c, const double *P, int skip) {
     const int order_carried[3] = {2, 0, 1}, order_plain[3] = {0, 1, 2}, order_div[3] = {1, 2, 0};
     const int *order = c->dmode && skip != 1 ? order_div : (c->carried ? order_carried : order_plain);
     // small grids: x and y in one launch (and z, where the x faces do not need what it stores)
-    const bool merge = !c->shared_edges && face_count(c->g, 0) < MERGE_FACES, merge_z = merge && c->nb == 9 && !c->carried;
+    const bool merge = !c->shared_edges && face_count(c->g, 0) < merge_faces(c->nb == 9, l.recon, l.mixed);
+    const bool merge_z = merge && c->nb == 9 && !c->carried;
     FaceLaunch d3[3] = {l, l, l};
     bool first = true;
     for (int n = 0; n < 3; ++n) {

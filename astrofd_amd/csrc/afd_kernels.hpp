@@ -328,12 +328,9 @@ template <int RECON, int RIEM, int DIR, typename T>
 __global__ __launch_bounds__(BLOCK) void k_face_srhd(FaceArgs<T> a) {
     face_srhd<RECON, RIEM, DIR, T>(a, blockIdx.x, gridDim.x);
 }
-// Several directions' faces in one launch (x first, nx workgroups, then y and z): below MERGE_FACES faces
-// a direction's waves are a few rounds of what the chip holds, or less than one, so that each launch ends in
-// a round that leaves most of it idle.  Faces of a step (SSPRK3), launches of their own and merged: SRHD MUSCL
-// FP64 48^3 0.063 -> 0.044 ms, 128^3 0.332 -> 0.298; RMHD WENO5 FP64 48^3 0.170 -> 0.150, 128^3 2.00 -> 1.95;
-// RMHD MUSCL FP64 80^3 0.333 -> 0.268, 150^3 2.02 -> 1.97.
-constexpr long MERGE_FACES = 3l << 20;
+// Several directions' faces in one launch (x first, nx workgroups, then y and z): on small grids a direction's
+// waves are a few rounds of what the chip holds, or less than one, so that each launch ends in a round that
+// leaves most of it idle.  Which grids: merge_faces.
 template <int RECON, int RIEM, typename T>
 __global__ __launch_bounds__(BLOCK) void k_faces_srhd(FaceArgs<T> x, FaceArgs<T> y, unsigned nx) {
     if (blockIdx.x < nx) face_srhd<RECON, RIEM, 0, T>(x, blockIdx.x, nx);

@@ -52,6 +52,24 @@ inline long face_count(const Grid &g, int dir) {
     return n;
 }
 
+// SRHD MUSCL x and y faces go by runs (afd_srhd.hip) from RUN_FACES faces on, in one launch of one thread a face
+// below.  Step (SSPRK2, HLLC) by runs over the merged launch, FP64 and mixed: 96^3 1.08 and 1.12, 128^3 (2.1 million
+// faces) 1.00 and 1.01, 90 x 90 x 300 (2.5) 1.02 and 1.01, 144^3 (3.0) 1.01 and 0.99, 150^3 (3.4) 0.98 and 0.97,
+// 152^3 (3.5) 0.96 and 0.95, 192^3 (7.1) 0.95 and 0.92; HLLE FP64 1.02 at 128^3, 1.00 at 144^3, 0.99 at 152^3.
+constexpr long RUN_FACES = 3l << 20;
+
+// The other schemes' directions share a launch below this many x faces.  Step (SSPRK2) merged over a launch each:
+// RMHD FP64 MUSCL 0.82 at 64^3, 0.98 at 128^3, 0.987 at 150^3 (3.4 million faces), 0.992 at 168^3 (4.8), 0.994 to
+// 0.998 above; PPM, where z stays by itself, 0.91, 0.987, 0.995 and 0.994, 1.00 at 224^3; WENO5 0.93, 0.987, 0.998
+// and 0.999, 1.00 above; mixed PPM 0.89, 0.985, 0.997 and 0.996, above 0.995 to 1.00.  Mixed RMHD MUSCL loses from
+// four million on: 0.87, 0.98, 0.98, 1.007 at 160^3 and 168^3, 1.02 at 176^3.  SRHD FP64 PPM 0.89 at 64^3, 0.97 at 152^3
+// (3.5), 1.01 at 168^3 and 176^3, 1.00 at 256^3; WENO5 0.90, 0.98, 0.995 and 0.99, 1.00; mixed 0.89 to 0.90, 0.97 to 0.98,
+// 0.97 to 0.99, 1.00.  (Medians of paired bursts, quartiles within 0.01.)
+inline long merge_faces(bool rmhd, int recon, bool mixed) {
+    if (recon == 0 && !rmhd) return RUN_FACES;
+    return recon == 0 && mixed ? 7l << 19 : 9l << 19;
+}
+
 // The faces of one direction; y, z not null: l's (x) faces with those in one launch (k_faces_srhd, k_faces_rmhd).
 hipError_t launch_face_srhd(const FaceLaunch &l, const FaceLaunch *y, hipStream_t s);
 hipError_t launch_face_rmhd(const FaceLaunch &l, const FaceLaunch *y, const FaceLaunch *z, hipStream_t s);

@@ -6,7 +6,7 @@
 
 namespace afd {
 
-// MUSCL faces go by runs from MERGE_FACES faces on; SLOTS waves of them run at a time (four on each of the
+// MUSCL faces go by runs from RUN_FACES faces on; SLOTS waves of them run at a time (four on each of the
 // 1024 SIMDs), and the length is the one whose rounds of waves take the fewest face times, a run's start
 // counted as START of them (RUN_MAX: longer runs gain nothing and leave the L2s).
 constexpr long RUN_MAX = 32, SLOTS = 4096;
@@ -36,7 +36,7 @@ template <int RECON, int RIEM, typename T> static void go(const FaceLaunch &l, c
         return;
     }
     if constexpr (RECON == 0) {
-        if (count >= MERGE_FACES) {
+        if (count >= RUN_FACES) {
             const int faces = g.r1[l.dir] - g.r0[l.dir] + 1;
             const long npos = count / faces, nb = (npos + BLOCK - 1) / BLOCK;
             const int run = run_length(npos, faces);

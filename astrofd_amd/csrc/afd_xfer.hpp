@@ -11,9 +11,9 @@ namespace afd {
 void xfer_retain();
 void xfer_release();
 
-// A context's own pinned block of PIN_BLOCK bytes (null: none to be had, or none free and `lock` false).  Closed contexts leave up to
-// two for the next ones (a fresh one takes 10 us a page-locked allocation, which a caller that opens a
-// context for each small step would pay each time); the last reference gives them back.
+// A context's own pinned block of PIN_BLOCK bytes (null: none to be had, or none free and `lock` false).
+// Closed contexts leave up to two for the next ones (locking and unlocking one takes 30 us, which a caller
+// that opens contexts beside one it holds would pay each time); the last reference gives them back.
 constexpr size_t PIN_BYTES = size_t(512) << 10, PIN_BLOCK = 2 * PIN_BYTES + 4096;
 char *xfer_pin_get(bool lock);
 void xfer_pin_put(char *block);
